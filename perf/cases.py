@@ -57,7 +57,7 @@ def listed():
     """Twelve cases; the sizes are the benchmark's own where it has the call."""
     named = {
         # a column of 32-bit keys, resident in HBM: the benchmark's 64 MiB RLE v1 decode
-        "rlev1_decode_64MiB": _case("rlev1_decode", 64 * MIB, 128 * KIB, 4, 32, known=True),
+        "rlev1_decode_64MiB": _case("rlev1_decode", 64 * MIB, 128 * KIB, 4, 128, known=True),
         # the drop-in call of a program that holds a container file in host memory
         "rlev1_host_16MiB": _case("rlev1_host", 16 * MIB, 128 * KIB, 4, 32),
         # one request of three chunks, the last one cut short: latency
@@ -75,7 +75,7 @@ def listed():
         # ordered by compressed size for the persistent launch
         "inflate_2048_streams": _case("inflate", 1200 * MIB, 4 * MIB, count=2048, sched=True, verify=False),
         # encode of each codec, resident in HBM: a table being written
-        "rlev1_encode_64MiB": _case("rlev1_encode", 64 * MIB, 128 * KIB, 4, 32),
+        "rlev1_encode_64MiB": _case("rlev1_encode", 64 * MIB, 128 * KIB, 4, 128),
         "rlev2_encode_256MiB": _case("rlev2_encode", 256 * MIB, 128 * KIB, 8, 512),
         "brle_encode_64MiB": _case("brle_encode", 64 * MIB, 256 * KIB),
         "lzss_encode_64MiB": _case("lzss_encode", 64 * MIB, 64 * KIB),
