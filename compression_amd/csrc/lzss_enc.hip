@@ -6,15 +6,27 @@
 // interleave :497-509).  Payload, col_len, col_map and blk_off equal that
 // encoder's output byte for byte.
 //
-// One wave per chunk; lane t < 32 encodes lane stream t (chunk bytes
-// 128 k + 4 t + j, j < 4) greedily: at each position the longest match of
-// 3..34 bytes within the lane's last 2048 bytes, ties to the oldest, else a
-// literal; tokens in groups of 8 behind a flag byte.  Matches are found
-// through hash chains over 3-byte prefixes: chain heads (u16) in LDS, chain
-// links in the work buffer; every candidate's length is measured, so the
-// choice equals the oldest-first window scan's.  The wave then ranks the 32
-// lanes by length (descending, ties to the higher lane id) into col_map, and
-// the shared kernels scan the chunk lengths and interleave the sorted lanes.
+// Lane stream t of a chunk is chunk bytes 128 k + 4 t + j (j < 4).  It is
+// encoded greedily: at each position the longest match of 3..34 bytes within
+// the last 2047 bytes (never from position 0), ties to the oldest, else a
+// literal; tokens in groups of 8 behind a flag byte.
+//
+// Half a wave encodes one lane stream, so a wave takes two neighbouring
+// lanes and both share each instruction.  The stream's bytes and an index of
+// its positions live in LDS: `slot` lists the positions bucket by bucket (9
+// hash bits of 3 bytes), ascending inside a bucket.  At each token the 32
+// lanes of the half compare 32 candidates of the token's bucket at once,
+// oldest first, and a maximum over (length, age) picks the match; a search
+// ends when no younger candidate can be longer.  Only the positions the
+// greedy parse reaches are searched.  What bounds it is the dependent chain
+// of LDS reads from one token to the next, so what counts is how many
+// streams a CU holds: 7.2 KiB of LDS each up to 2048 lane bytes (64 KiB
+// chunks), 13.4 KiB beyond.  Lanes over 4096 bytes are indexed in windows of
+// 4096 positions that advance by 2048.
+//
+// A second kernel ranks a chunk's 32 lanes by length (descending, ties to
+// the higher lane id) into col_map; the shared kernels scan the chunk
+// lengths and interleave the sorted lanes.
 #include "lanes_enc_dev.h"
 #include "mdz_device.h"
 #include "mdz_internal.h"
@@ -23,126 +35,255 @@ namespace mdz {
 namespace {
 
 constexpr uint32_t kHist = 2048, kMinLen = 3, kMaxLen = 34, kLenBits = 5;
-constexpr uint32_t kHashBits = 8, kNoPos = 0xFFFF;
+constexpr uint32_t kHashBits = 9, kBuckets = 1u << kHashBits;
+constexpr uint32_t kHalf = 32;                  // lanes that encode one stream
+constexpr uint32_t kPairs = 16;                 // neighbouring lane pairs of a chunk
+constexpr uint32_t kXcds = 8;
 
-struct LzEncLds {
-    uint16_t head[32][1u << kHashBits];
-    uint64_t len[32];
+// One lane stream's window: kCap positions and the bytes a match at the last
+// of them can reach.
+template <uint32_t kCap>
+struct LzStream {
+    static constexpr bool kOld = kCap > kHist;  // candidates can be out of reach
+    uint32_t data[(kCap + 64) / 4];
+    uint16_t slot[kCap];                        // positions by bucket, ascending
+    uint32_t end[kBuckets / 2];                 // u16 pairs: one past a bucket's last slot
+    uint16_t first[kOld ? kBuckets : 2];        // first slot still within reach
 };
 
-struct LaneSrc {
-    const uint8_t* chunk;
-    uint32_t t;
-    uint32_t nd;                                 // lane dwords (lane bytes / 4)
-    MDZ_DEV uint32_t at(uint32_t i) const { return chunk[128u * (i >> 2) + 4u * t + (i & 3u)]; }
-    // lane bytes i..i+3 (zero past the lane's end): two aligned dwords of the
-    // lane's rows, shifted together
-    MDZ_DEV uint32_t dword(uint32_t k) const {
-        return k < nd ? *reinterpret_cast<const uint32_t*>(chunk + 128u * k + 4u * t) : 0u;
-    }
-    MDZ_DEV uint32_t word_at(uint32_t i) const {
-        const uint32_t k = i >> 2, sh = i & 3u, lo = dword(k);
-        return sh ? alignbyte(dword(k + 1), lo, sh) : lo;
-    }
-    MDZ_DEV uint32_t hash3(uint32_t i) const {          // lane bytes i, i+1, i+2
-        const uint32_t v = word_at(i) & 0xFFFFFFu;
-        return (v * 2654435761u) >> (32 - kHashBits);
-    }
-};
+MDZ_DEV uint32_t lds_u32(const uint8_t* p) {    // any alignment
+    uint32_t v;
+    __builtin_memcpy(&v, p, 4);
+    return v;
+}
+MDZ_DEV uint32_t lz_hash(uint32_t v) { return ((v & 0xFFFFFFu) * 2654435761u) >> (32 - kHashBits); }
 
-MDZ_DEV uint64_t encode_lzss_lane(const LaneSrc& s, uint32_t n, uint16_t* head, uint16_t* prev, uint8_t* out) {
-    for (uint32_t h = 0; h < (1u << kHashBits); ++h) head[h] = (uint16_t)kNoPos;
-    auto insert = [&](uint32_t p) {
-        if (p + kMinLen > n) return;
-        const uint32_t h = s.hash3(p);
-        prev[p] = head[h];
-        head[h] = (uint16_t)p;
-    };
-    uint64_t o = 1, flag_at = 0;
-    uint32_t ntok = 0, flags = 0;
-    out[0] = 0;
-    for (uint32_t cur = 0; cur < n;) {
-        // the longest match of the window, ties to the oldest
-        uint32_t best = 0, best_q = 0;
-        if (n - cur >= kMinLen && cur >= 2) {
-            const uint32_t count = cur < kHist ? cur : kHist;
-            const uint32_t lo = cur - count + 1;
-            const uint32_t look = n - cur;
-            for (uint32_t q = head[s.hash3(cur)]; q != kNoPos && q >= lo; q = prev[q]) {
-                uint32_t cap = min(cur - q, look);
-                cap = cap < kMaxLen ? cap : kMaxLen;
-                uint32_t f = 0;                  // common prefix, four bytes at a time
-                while (f < cap) {
-                    const uint32_t x = s.word_at(q + f) ^ s.word_at(cur + f);
-                    if (x) {
-                        f += (uint32_t)__builtin_ctz(x) >> 3;
-                        break;
-                    }
-                    f += 4;
-                }
-                f = f < cap ? f : cap;
-                if (f >= best) {
-                    best = f;
-                    best_q = q;
-                }
-            }
-        }
-        if (best < kMinLen) {
-            flags |= 1u << ntok;
-            out[o++] = (uint8_t)s.at(cur);
-            insert(cur);
-            cur += 1;
-        } else {
-            const uint32_t v = ((cur - best_q) << kLenBits) | (best - kMinLen);
-            out[o] = (uint8_t)v;
-            out[o + 1] = (uint8_t)(v >> 8);
-            o += 2;
-            for (uint32_t i = 0; i < best; ++i) insert(cur + i);
-            cur += best;
-        }
-        if (++ntok == 8) {                      // the next group's flag byte is reserved at once
-            out[flag_at] = (uint8_t)flags;
-            flags = 0;
-            ntok = 0;
-            flag_at = o++;
-            out[flag_at] = 0;
-        }
-    }
-    if (ntok) out[flag_at] = (uint8_t)flags;
-    return o;
+// Maximum over each half of the wave, in every lane of the half.
+MDZ_DEV uint32_t half_max_u32(uint32_t v) {
+    v = max(v, dpp_src<0x128, 0xf, 0u>(v));     // row_ror 8, 4, 2, 1: each row of 16
+    v = max(v, dpp_src<0x124, 0xf, 0u>(v));
+    v = max(v, dpp_src<0x122, 0xf, 0u>(v));
+    v = max(v, dpp_src<0x121, 0xf, 0u>(v));
+    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return max(r[0], r[1]);                     // rows 0 and 1, rows 2 and 3
+}
+MDZ_DEV uint32_t half_incl_scan_u32(uint32_t v) {
+    v += dpp_src<0x111, 0xf, 0u>(v);
+    v += dpp_src<0x112, 0xf, 0u>(v);
+    v += dpp_src<0x114, 0xf, 0u>(v);
+    v += dpp_src<0x118, 0xf, 0u>(v);
+    v += dpp_src<0x142, 0xa, 0u>(v);            // row_bcast:15 into rows 1 and 3
+    return v;
+}
+// The half's 32 bits of a ballot.
+MDZ_DEV uint32_t half_ballot(bool b) {
+    const uint64_t m = __ballot(b);
+    return lane_id() < kHalf ? (uint32_t)m : (uint32_t)(m >> 32);
 }
 
-__global__ __launch_bounds__(kWave) void lzss_encode_kernel(const uint8_t* __restrict__ in, uint64_t chunk,
-                                                            uint64_t lane_slot, uint8_t* __restrict__ work,
-                                                            uint16_t* __restrict__ links,
-                                                            uint64_t* __restrict__ col_len,
-                                                            uint8_t* __restrict__ col_map,
-                                                            uint64_t* __restrict__ chunk_len) {
-    __shared__ LzEncLds S;
-    const uint32_t l = lane_id();
-    const uint64_t c = blockIdx.x;
-    const uint32_t lb = (uint32_t)(chunk / 32);
-    if (l < 32) {
-        const LaneSrc src{in + c * chunk, l, lb / 4};
-        S.len[l] = encode_lzss_lane(src, lb, S.head[l], links + (c * 32 + l) * lb,
-                                    work + (c * 32 + l) * lane_slot);
+// Lists the window's positions [p0, p1) by bucket.  All 64 lanes; each half
+// builds its own stream's index.
+template <uint32_t kCap>
+MDZ_DEV void lz_index(LzStream<kCap>& S, uint32_t p0, uint32_t p1, uint32_t sub) {
+    const uint8_t* bytes = reinterpret_cast<const uint8_t*>(S.data);
+    for (uint32_t i = sub; i < kBuckets / 2; i += kHalf) S.end[i] = 0;
+    wave_sync();
+    for (uint32_t p = p0 + sub; p < p1; p += kHalf) {
+        const uint32_t h = lz_hash(lds_u32(bytes + p));
+        atomicAdd(&S.end[h >> 1], 1u << (16 * (h & 1)));
     }
     wave_sync();
-    // sorted slot of lane t: longer lanes first, equal lengths by higher lane id
-    uint32_t words = 0;
-    if (l < 32) {
-        const uint64_t mine = S.len[l];
-        uint32_t rank = 0;
-        for (uint32_t u = 0; u < 32; ++u) {
-            const uint64_t other = S.len[u];
-            rank += (other > mine || (other == mine && u > l)) ? 1u : 0u;
+    {   // counts -> first slots, 16 buckets a lane
+        constexpr uint32_t kPer = kBuckets / 2 / kHalf;
+        uint32_t c[kPer], sum = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kPer; ++i) {
+            c[i] = S.end[sub * kPer + i];
+            sum += (c[i] & 0xFFFFu) + (c[i] >> 16);
         }
-        col_len[c * 32 + rank] = mine;
-        col_map[c * 32 + rank] = (uint8_t)l;
-        words = (uint32_t)((mine + 3) / 4);
+        uint32_t at = half_incl_scan_u32(sum) - sum;
+#pragma unroll
+        for (uint32_t i = 0; i < kPer; ++i) {
+            const uint32_t lo = at, hi = at + (c[i] & 0xFFFFu);
+            at = hi + (c[i] >> 16);
+            S.end[sub * kPer + i] = lo | hi << 16;
+            if constexpr (LzStream<kCap>::kOld) {
+                S.first[2 * (sub * kPer + i)] = (uint16_t)lo;
+                S.first[2 * (sub * kPer + i) + 1] = (uint16_t)hi;
+            }
+        }
     }
-    const uint32_t total = wave_sum_u32(words);
-    if (l == 0) chunk_len[c] = ((uint64_t)total * 4 + 127) / 128 * 128;
+    wave_sync();
+    for (uint32_t p = p0 + sub; p < p1; p += kHalf) {   // each slot taken moves its bucket's end
+        const uint32_t h = lz_hash(lds_u32(bytes + p));
+        const uint32_t at = atomicAdd(&S.end[h >> 1], 1u << (16 * (h & 1)));
+        S.slot[(at >> (16 * (h & 1))) & 0xFFFFu] = (uint16_t)p;
+    }
+    wave_sync();
+    // The 32 positions of one step may take their bucket's slots in any
+    // order: put neighbours in order until none is out of it.
+    const uint32_t ns = p1 > p0 ? p1 - p0 : 0;
+    for (;;) {
+        bool moved = false;
+#pragma unroll
+        for (uint32_t odd = 0; odd < 2; ++odd) {
+            for (uint32_t i = odd + 2 * sub; i + 1 < ns; i += 2 * kHalf) {
+                const uint32_t a = S.slot[i], b = S.slot[i + 1];
+                if (a > b && lz_hash(lds_u32(bytes + a)) == lz_hash(lds_u32(bytes + b))) {
+                    S.slot[i] = (uint16_t)b;
+                    S.slot[i + 1] = (uint16_t)a;
+                    moved = true;
+                }
+            }
+            wave_sync();
+        }
+        if (!__ballot(moved)) break;
+    }
+}
+
+template <uint32_t kCap>
+__global__ __launch_bounds__(kWave) void lzss_encode_kernel(const uint8_t* __restrict__ in, uint64_t n_chunks,
+                                                            uint64_t chunk, uint64_t lane_slot,
+                                                            uint8_t* __restrict__ work,
+                                                            uint32_t* __restrict__ lane_len) {
+    __shared__ LzStream<kCap> streams[2];
+    const uint32_t l = lane_id(), sub = l & (kHalf - 1), half = l / kHalf;
+    LzStream<kCap>& S = streams[half];
+    const uint8_t* bytes = reinterpret_cast<const uint8_t*>(S.data);
+    const uint16_t* ends = reinterpret_cast<const uint16_t*>(S.end);
+    const uint32_t n = (uint32_t)(chunk / 32);
+    // A chunk's 16 pairs read the same 128-byte rows: they run on one XCD
+    // (workgroups go to the XCDs in turn), so its L2 reads each row once.
+    const uint64_t units = (n_chunks + kXcds - 1) / kXcds * kXcds * kPairs;
+    for (uint64_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
+        const uint32_t pair = (uint32_t)(unit / kXcds) % kPairs;
+        const uint64_t c = unit / (kXcds * kPairs) * kXcds + unit % kXcds;
+        if (c >= n_chunks) continue;
+        const uint8_t* rows = in + c * chunk + 8 * pair;
+        const uint64_t lane = c * 32 + 2 * pair + half;
+        uint8_t* out = work + lane * lane_slot;
+        uint32_t o = 1, flag_at = 0, ntok = 0, flags = 0;
+        uint32_t cur = 0;                       // next position, counted from the window's start
+        for (uint32_t w0 = 0;; w0 += kHist) {
+            const uint32_t stop = min(n - w0, kCap);    // positions of the window
+            wave_sync();
+            for (uint32_t k = l; k < (kCap + 64) / 4; k += kWave) {
+                uint32_t v[2] = {0, 0};
+                if (w0 / 4 + k < n / 4) __builtin_memcpy(v, __builtin_assume_aligned(rows + 128ull * (w0 / 4 + k), 4), 8);
+                streams[0].data[k] = v[0];
+                streams[1].data[k] = v[1];
+            }
+            wave_sync();
+            // position 0 is never a candidate, nor one with under 3 bytes left
+            const uint32_t p0 = w0 ? 0u : 1u, left = n - w0;
+            lz_index<kCap>(S, p0, min(stop, left >= kMinLen ? left - (kMinLen - 1) : 0u), sub);
+            while (__ballot(cur < stop)) {
+                const bool on = cur < stop;
+                const uint32_t at = on ? cur : 0;
+                const uint32_t word = lds_u32(bytes + at);
+                const uint32_t h = lz_hash(word);
+                const uint32_t look = on ? min(left - at, kMaxLen) : 0;    // longest match left
+                const uint32_t lo = at >= kHist ? at - kHist + 1 : 0;
+                uint32_t i, e = look >= kMinLen ? ends[h] : 0;
+                if constexpr (LzStream<kCap>::kOld) i = S.first[h];
+                else i = h ? ends[h - 1] : 0;
+                uint32_t key = 0;               // length << 16 | 0xFFFF - position
+                while (__ballot(i < e)) {
+                    const uint32_t best = key >> 16;
+                    const uint32_t q = i + sub < e ? S.slot[i + sub] : 0xFFFFu;
+                    bool live = q < at && q >= lo;
+                    const uint32_t cap = live ? min(at - q, look) : 0;
+                    // a better match agrees on the byte after the best one's
+                    // last, and on the two before it
+                    const uint32_t probe = best >= kMinLen ? best - (kMinLen - 1) : 0;
+                    live = live && cap > best;
+                    const uint32_t qa = live ? q : 0;
+                    const uint32_t x = lds_u32(bytes + qa + probe) ^ lds_u32(bytes + at + probe);
+                    live = live && (x & 0xFFFFFFu) == 0;
+                    uint32_t f = 0;
+                    if (__ballot(live)) {
+                        bool run = live;
+                        while (__ballot(run)) {  // 8 bytes at a time
+                            const uint32_t fa = run ? f : 0, qf = run ? q : 0;
+                            uint64_t a, b;
+                            __builtin_memcpy(&a, bytes + qf + fa, 8);
+                            __builtin_memcpy(&b, bytes + at + fa, 8);
+                            a ^= b;
+                            f = !run ? f : a ? f + ((uint32_t)__builtin_ctzll(a) >> 3) : f + 8;
+                            run = run && !a && f < cap;
+                        }
+                        f = min(f, cap);
+                        const uint32_t mine = live && f > best && f >= kMinLen ? f << 16 | (0xFFFFu - q) : 0u;
+                        key = max(key, half_max_u32(mine));
+                    }
+                    if constexpr (LzStream<kCap>::kOld) {
+                        // a step wholly out of reach stays so for later positions
+                        if (on && i + kHalf <= e && half_ballot(q < lo) == 0xFFFFFFFFu && sub == 0)
+                            S.first[h] = (uint16_t)(i + kHalf);
+                    }
+                    i += kHalf;
+                    // younger candidates: none, past the position, or too near to be longer
+                    const uint32_t got = key >> 16;
+                    const uint32_t reach = half_max_u32(q < at ? q : i - kHalf + sub < e ? 0xFFFFu : 0u);
+                    if (got >= look || reach >= at || at - reach <= got) i = e;
+                }
+                if (on) {
+                    const uint32_t len = key >> 16;
+                    if (len == 0) {
+                        if (sub == 0) out[o] = (uint8_t)word;
+                        flags |= 1u << ntok;
+                        o += 1;
+                        cur += 1;
+                    } else {
+                        const uint32_t dist = at - (0xFFFFu - (key & 0xFFFFu));
+                        const uint16_t v = (uint16_t)(dist << kLenBits | (len - kMinLen));
+                        if (sub == 0) __builtin_memcpy(out + o, &v, 2);
+                        o += 2;
+                        cur += len;
+                    }
+                    if (++ntok == 8) {          // the next group's flag byte is reserved at once
+                        if (sub == 0) out[flag_at] = (uint8_t)flags;
+                        flags = 0;
+                        ntok = 0;
+                        flag_at = o++;
+                    }
+                }
+                if constexpr (LzStream<kCap>::kOld) wave_sync();    // first[] before its next reader
+            }
+            if (stop == left) break;
+            cur -= kHist;                       // the next window starts kHist positions on
+        }
+        if (sub == 0) {
+            out[flag_at] = (uint8_t)flags;
+            lane_len[lane] = o;
+        }
+    }
+}
+
+// Sorted slot of lane t: longer lanes first, equal lengths by higher lane id.
+// Half a wave per chunk.
+constexpr uint32_t kRankThreads = 256, kRankChunks = kRankThreads / kHalf;
+
+__global__ __launch_bounds__(kRankThreads) void lzss_rank_kernel(const uint32_t* __restrict__ lane_len, uint64_t n_chunks,
+                                                                 uint64_t* __restrict__ col_len,
+                                                                 uint8_t* __restrict__ col_map,
+                                                                 uint64_t* __restrict__ chunk_len) {
+    __shared__ uint32_t len[kRankThreads];
+    const uint32_t t = threadIdx.x % kHalf;
+    const uint64_t c = (uint64_t)blockIdx.x * kRankChunks + threadIdx.x / kHalf;
+    const uint32_t mine = c < n_chunks ? lane_len[c * 32 + t] : 0u;
+    len[threadIdx.x] = mine;
+    wave_sync();
+    uint32_t rank = 0, words = 0;
+    for (uint32_t u = 0; u < kHalf; ++u) {
+        const uint32_t other = len[threadIdx.x - t + u];
+        rank += (other > mine || (other == mine && u > t)) ? 1u : 0u;
+        words += (other + 3) / 4;
+    }
+    if (c >= n_chunks) return;
+    col_len[c * 32 + rank] = mine;
+    col_map[c * 32 + rank] = (uint8_t)t;
+    if (t == 0) chunk_len[c] = ((uint64_t)words * 4 + 127) / 128 * 128;
 }
 
 uint64_t lz_lane_slot(uint64_t chunk) {
@@ -174,12 +315,18 @@ int lzss_compress(const void* in, uint64_t in_bytes, uint64_t chunk, void* work,
     if ((uintptr_t)in & 3) return MDZ_ERR_INVALID;   // lanes are read a dword at a time
     const uint64_t slot = lz_lane_slot(chunk);
     uint8_t* w = static_cast<uint8_t*>(work);
-    uint16_t* links = reinterpret_cast<uint16_t*>(w + n * 32 * slot);
+    uint32_t* lane_len = reinterpret_cast<uint32_t*>(w + n * 32 * slot);
     uint64_t* chunk_len = reinterpret_cast<uint64_t*>(w + n * 32 * slot + n * chunk * 2);
-    hipLaunchKernelGGL(lzss_encode_kernel, dim3((uint32_t)n), dim3(kWave), 0, s, static_cast<const uint8_t*>(in),
-                       chunk, slot, w, links, col_len, col_map, chunk_len);
+    const uint32_t lb = (uint32_t)(chunk / 32);
+    const uint64_t units = (n + kXcds - 1) / kXcds * kXcds * kPairs;
+    const dim3 grid((uint32_t)(units < (1u << 24) ? units : 1u << 24)), block(kWave);
+    auto encode = lb <= 1024 ? lzss_encode_kernel<1024> : lb <= 2048 ? lzss_encode_kernel<2048> : lzss_encode_kernel<4096>;
+    hipLaunchKernelGGL(encode, grid, block, 0, s, static_cast<const uint8_t*>(in), n, chunk, slot, w, lane_len);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return record_hip(e, "lzss_encode_kernel launch");
+    hipLaunchKernelGGL(lzss_rank_kernel, dim3((uint32_t)((n + kRankChunks - 1) / kRankChunks)), dim3(kRankThreads), 0, s,
+                       lane_len, n, col_len, col_map, chunk_len);
+    if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lzss_rank_kernel launch");
     hipLaunchKernelGGL(lanes_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, chunk_len, n, blk_off, nullptr, ~0ull);
     if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lanes_scan_kernel launch");
     hipLaunchKernelGGL(lanes_interleave_kernel, dim3((uint32_t)n), dim3(kIlvThreads), 0, s,

@@ -48,3 +48,29 @@ def test_host_form_roundtrip(gpu):
     assert blobs[0] == np.uint64(131072).tobytes() and blobs[1] == ref.blk_off.tobytes()
     assert blobs[2] == ref.col_len.tobytes() and blobs[3] == ref.col_map.tobytes()
     assert lzss.decompress_gpu(payload, blobs) == data[:5 * 131072].tobytes()
+
+
+# lane bytes at the edges of the encoder's LDS windows (1024, 2048, 4096
+# positions), the windows that advance by 2048 above, and the smallest lanes
+@pytest.mark.parametrize("lane_bytes", [4, 8, 40, 1024, 1028, 2044, 2048, 2052, 4096, 4100, 6144, 10240, 32768])
+def test_window_edges(gpu, lane_bytes):
+    from compression_amd import lzss
+    from compression_amd._lib import DeviceBuffer
+    chunk = 32 * lane_bytes
+    size = max(3 * chunk, min(20 * chunk, 400_000))
+    rng = np.random.default_rng(lane_bytes)
+    far = np.zeros(size, np.uint8)                 # matches at the far end of the history
+    far[:] = np.tile(rng.integers(0, 256, 2045 * 32), -(-size // (2045 * 32)))[:size]
+    for name, data in {"markov": host.gen_lzss_markov(size, lane_bytes), "far": far,
+                       "pairs": rng.integers(0, 2, size).astype(np.uint8),
+                       "zeros": np.zeros(size, np.uint8)}.items():
+        n, wb, cap = lzss.compress_bound(size, chunk)
+        src, work, pay = DeviceBuffer.from_array(data), DeviceBuffer(wb), DeviceBuffer(cap)
+        col, cmap, off = DeviceBuffer(256 * n), DeviceBuffer(32 * n), DeviceBuffer(8 * (n + 1))
+        print(f"lzss encode {name} lane_bytes={lane_bytes} n={n}", flush=True)
+        lzss.compress(src, size, chunk, work, pay, col, cmap, off)
+        ref = host.lzss_encode(data, chunk)
+        assert np.array_equal(off.download(8 * (n + 1)).view(np.uint64), ref.blk_off), name
+        assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len), name
+        assert np.array_equal(cmap.download(32 * n), ref.col_map), name
+        assert pay.download(int(ref.blk_off[-1])).tobytes() == ref.payload[:int(ref.blk_off[-1])].tobytes(), name
