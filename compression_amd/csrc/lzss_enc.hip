@@ -11,18 +11,19 @@
 // the last 2047 bytes (never from position 0), ties to the oldest, else a
 // literal; tokens in groups of 8 behind a flag byte.
 //
-// Half a wave encodes one lane stream, so a wave takes two neighbouring
-// lanes and both share each instruction.  The stream's bytes and an index of
-// its positions live in LDS: `slot` lists the positions bucket by bucket (9
-// hash bits of 3 bytes), ascending inside a bucket.  At each token the 32
-// lanes of the half compare 32 candidates of the token's bucket at once,
-// oldest first, and a maximum over (length, age) picks the match; a search
-// ends when no younger candidate can be longer.  Only the positions the
-// greedy parse reaches are searched.  What bounds it is the dependent chain
-// of LDS reads from one token to the next, so what counts is how many
-// streams a CU holds: 7.2 KiB of LDS each up to 2048 lane bytes (64 KiB
-// chunks), 13.4 KiB beyond.  Lanes over 4096 bytes are indexed in windows of
-// 4096 positions that advance by 2048.
+// One wave encodes one lane stream.  The stream's bytes and an index of its
+// positions live in LDS: `slot` lists the positions bucket by bucket (9 hash
+// bits of 3 bytes), ascending inside a bucket.  At each token the 64 lanes
+// compare 64 candidates of the token's bucket at once, oldest first; a search
+// ends when no younger candidate can be longer.  Only the positions the greedy
+// parse reaches are searched, and what the whole wave shares (position, best
+// match, output offset) is scalar.  What bounds it is the dependent chain of
+// LDS reads and scalar steps from one token to the next, so what counts is how
+// many streams a CU holds: 7.4 KiB of LDS each up to 2048 lane bytes (64 KiB
+// chunks), 14 KiB beyond.  Lanes over 4096 bytes are indexed in windows of
+// 4096 positions that advance by 2048.  64 MiB in 64 KiB chunks: 3.4 ms, VALU
+// issue 66 % busy (412 ms with one lane per stream and chains in global
+// memory; 6.5 ms with half a wave per stream and misaligned LDS reads).
 //
 // A second kernel ranks a chunk's 32 lanes by length (descending, ties to
 // the higher lane id) into col_map; the shared kernels scan the chunk
@@ -36,8 +37,6 @@ namespace {
 
 constexpr uint32_t kHist = 2048, kMinLen = 3, kMaxLen = 34, kLenBits = 5;
 constexpr uint32_t kHashBits = 9, kBuckets = 1u << kHashBits;
-constexpr uint32_t kHalf = 32;                  // lanes that encode one stream
-constexpr uint32_t kPairs = 16;                 // neighbouring lane pairs of a chunk
 constexpr uint32_t kXcds = 8;
 
 // One lane stream's window: kCap positions and the bytes a match at the last
@@ -46,90 +45,78 @@ template <uint32_t kCap>
 struct LzStream {
     static constexpr bool kOld = kCap > kHist;  // candidates can be out of reach
     uint32_t data[(kCap + 64) / 4];
-    uint16_t slot[kCap];                        // positions by bucket, ascending
-    uint32_t end[kBuckets / 2];                 // u16 pairs: one past a bucket's last slot
+    uint16_t slot[kCap + kWave];                // positions by bucket, ascending (the tail is read, not used)
+    uint32_t bound[kBuckets / 2 + 1];           // u16: bucket h's slots are [bound[h], bound[h + 1])
     uint16_t first[kOld ? kBuckets : 2];        // first slot still within reach
 };
 
-MDZ_DEV uint32_t lds_u32(const uint8_t* p) {    // any alignment
-    uint32_t v;
-    __builtin_memcpy(&v, p, 4);
-    return v;
+// 4 and 8 bytes at byte p: whole dwords shifted together.  (A misaligned LDS
+// read is one instruction too, but serialises the wave's lanes: with those the
+// encoder spent 94 % of its time in LDS.)
+MDZ_DEV uint32_t lds_u32(const uint32_t* w, uint32_t p) {
+    const uint32_t k = p >> 2;
+    return alignbyte(w[k + 1], w[k], p & 3);
+}
+MDZ_DEV uint64_t lds_u64(const uint32_t* w, uint32_t p) {
+    const uint32_t k = p >> 2, w0 = w[k], w1 = w[k + 1], w2 = w[k + 2];
+    return (uint64_t)alignbyte(w2, w1, p & 3) << 32 | alignbyte(w1, w0, p & 3);
 }
 MDZ_DEV uint32_t lz_hash(uint32_t v) { return ((v & 0xFFFFFFu) * 2654435761u) >> (32 - kHashBits); }
-
-// Maximum over each half of the wave, in every lane of the half.
-MDZ_DEV uint32_t half_max_u32(uint32_t v) {
-    v = max(v, dpp_src<0x128, 0xf, 0u>(v));     // row_ror 8, 4, 2, 1: each row of 16
-    v = max(v, dpp_src<0x124, 0xf, 0u>(v));
-    v = max(v, dpp_src<0x122, 0xf, 0u>(v));
-    v = max(v, dpp_src<0x121, 0xf, 0u>(v));
-    const auto r = __builtin_amdgcn_permlane16_swap(v, v, false, false);
-    return max(r[0], r[1]);                     // rows 0 and 1, rows 2 and 3
-}
-MDZ_DEV uint32_t half_incl_scan_u32(uint32_t v) {
-    v += dpp_src<0x111, 0xf, 0u>(v);
-    v += dpp_src<0x112, 0xf, 0u>(v);
-    v += dpp_src<0x114, 0xf, 0u>(v);
-    v += dpp_src<0x118, 0xf, 0u>(v);
-    v += dpp_src<0x142, 0xa, 0u>(v);            // row_bcast:15 into rows 1 and 3
-    return v;
-}
-// The half's 32 bits of a ballot.
-MDZ_DEV uint32_t half_ballot(bool b) {
-    const uint64_t m = __ballot(b);
-    return lane_id() < kHalf ? (uint32_t)m : (uint32_t)(m >> 32);
+MDZ_DEV uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+MDZ_DEV uint32_t lane_value_at(uint32_t v, uint32_t lane) {
+    return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lane);
 }
 
-// Lists the window's positions [p0, p1) by bucket.  All 64 lanes; each half
-// builds its own stream's index.
+// Lists the window's positions [p0, p1) by bucket.
 template <uint32_t kCap>
-MDZ_DEV void lz_index(LzStream<kCap>& S, uint32_t p0, uint32_t p1, uint32_t sub) {
-    const uint8_t* bytes = reinterpret_cast<const uint8_t*>(S.data);
-    for (uint32_t i = sub; i < kBuckets / 2; i += kHalf) S.end[i] = 0;
+MDZ_DEV void lz_index(LzStream<kCap>& S, uint32_t p0, uint32_t p1, uint32_t l) {
+    // While the slots are given out, the u16 at h + 1 counts bucket h.
+    auto bump = [&](uint32_t h) {
+        return (atomicAdd(&S.bound[(h + 1) >> 1], 1u << (16 * ((h + 1) & 1))) >> (16 * ((h + 1) & 1))) & 0xFFFFu;
+    };
+    for (uint32_t i = l; i <= kBuckets / 2; i += kWave) S.bound[i] = 0;
     wave_sync();
-    for (uint32_t p = p0 + sub; p < p1; p += kHalf) {
-        const uint32_t h = lz_hash(lds_u32(bytes + p));
-        atomicAdd(&S.end[h >> 1], 1u << (16 * (h & 1)));
-    }
+    for (uint32_t p = p0 + l; p < p1; p += kWave) bump(lz_hash(lds_u32(S.data, p)));
     wave_sync();
-    {   // counts -> first slots, 16 buckets a lane
-        constexpr uint32_t kPer = kBuckets / 2 / kHalf;
+    {   // counts -> first slots: lane l holds the u16s [8 l, 8 l + 8); the last one is never read as a count
+        constexpr uint32_t kPer = kBuckets / 2 / kWave;
         uint32_t c[kPer], sum = 0;
 #pragma unroll
         for (uint32_t i = 0; i < kPer; ++i) {
-            c[i] = S.end[sub * kPer + i];
+            c[i] = S.bound[l * kPer + i];
             sum += (c[i] & 0xFFFFu) + (c[i] >> 16);
         }
-        uint32_t at = half_incl_scan_u32(sum) - sum;
+        // the u16 at h + 1 becomes bucket h's first slot: the counts before it
+        uint32_t at = wave_incl_scan_u32(sum) - sum;
 #pragma unroll
         for (uint32_t i = 0; i < kPer; ++i) {
             const uint32_t lo = at, hi = at + (c[i] & 0xFFFFu);
             at = hi + (c[i] >> 16);
-            S.end[sub * kPer + i] = lo | hi << 16;
+            S.bound[l * kPer + i] = lo | hi << 16;
             if constexpr (LzStream<kCap>::kOld) {
-                S.first[2 * (sub * kPer + i)] = (uint16_t)lo;
-                S.first[2 * (sub * kPer + i) + 1] = (uint16_t)hi;
+                if (l || i) S.first[2 * (l * kPer + i) - 1] = (uint16_t)lo;
+                S.first[2 * (l * kPer + i)] = (uint16_t)hi;
             }
+        }
+        if (l == kWave - 1) {
+            S.bound[kBuckets / 2] = at;
+            if constexpr (LzStream<kCap>::kOld) S.first[kBuckets - 1] = (uint16_t)at;
         }
     }
     wave_sync();
-    for (uint32_t p = p0 + sub; p < p1; p += kHalf) {   // each slot taken moves its bucket's end
-        const uint32_t h = lz_hash(lds_u32(bytes + p));
-        const uint32_t at = atomicAdd(&S.end[h >> 1], 1u << (16 * (h & 1)));
-        S.slot[(at >> (16 * (h & 1))) & 0xFFFFu] = (uint16_t)p;
-    }
+    // each slot given out moves its bucket's first slot: to the bucket's end
+    for (uint32_t p = p0 + l; p < p1; p += kWave) S.slot[bump(lz_hash(lds_u32(S.data, p)))] = (uint16_t)p;
     wave_sync();
-    // The 32 positions of one step may take their bucket's slots in any
+    // The 64 positions of one step may take their bucket's slots in any
     // order: put neighbours in order until none is out of it.
     const uint32_t ns = p1 > p0 ? p1 - p0 : 0;
     for (;;) {
         bool moved = false;
 #pragma unroll
         for (uint32_t odd = 0; odd < 2; ++odd) {
-            for (uint32_t i = odd + 2 * sub; i + 1 < ns; i += 2 * kHalf) {
+            for (uint32_t i = odd + 2 * l; i + 1 < ns; i += 2 * kWave) {
                 const uint32_t a = S.slot[i], b = S.slot[i + 1];
-                if (a > b && lz_hash(lds_u32(bytes + a)) == lz_hash(lds_u32(bytes + b))) {
+                if (a > b && lz_hash(lds_u32(S.data, a)) == lz_hash(lds_u32(S.data, b))) {
                     S.slot[i] = (uint16_t)b;
                     S.slot[i + 1] = (uint16_t)a;
                     moved = true;
@@ -146,123 +133,98 @@ __global__ __launch_bounds__(kWave) void lzss_encode_kernel(const uint8_t* __res
                                                             uint64_t chunk, uint64_t lane_slot,
                                                             uint8_t* __restrict__ work,
                                                             uint32_t* __restrict__ lane_len) {
-    __shared__ LzStream<kCap> streams[2];
-    const uint32_t l = lane_id(), sub = l & (kHalf - 1), half = l / kHalf;
-    LzStream<kCap>& S = streams[half];
-    const uint8_t* bytes = reinterpret_cast<const uint8_t*>(S.data);
-    const uint16_t* ends = reinterpret_cast<const uint16_t*>(S.end);
+    __shared__ LzStream<kCap> S;
+    const uint32_t l = lane_id();
+    const uint16_t* bounds = reinterpret_cast<const uint16_t*>(S.bound);
     const uint32_t n = (uint32_t)(chunk / 32);
-    // A chunk's 16 pairs read the same 128-byte rows: they run on one XCD
+    // A chunk's 32 lanes read the same 128-byte rows: they run on one XCD
     // (workgroups go to the XCDs in turn), so its L2 reads each row once.
-    const uint64_t units = (n_chunks + kXcds - 1) / kXcds * kXcds * kPairs;
+    const uint64_t units = (n_chunks + kXcds - 1) / kXcds * kXcds * 32;
     for (uint64_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
-        const uint32_t pair = (uint32_t)(unit / kXcds) % kPairs;
-        const uint64_t c = unit / (kXcds * kPairs) * kXcds + unit % kXcds;
+        const uint32_t t = (uint32_t)(unit / kXcds) % 32;
+        const uint64_t c = unit / (kXcds * 32) * kXcds + unit % kXcds;
         if (c >= n_chunks) continue;
-        const uint8_t* rows = in + c * chunk + 8 * pair;
-        const uint64_t lane = c * 32 + 2 * pair + half;
-        uint8_t* out = work + lane * lane_slot;
+        const uint8_t* rows = in + c * chunk + 4 * t;
+        uint8_t* out = work + (c * 32 + t) * lane_slot;
         uint32_t o = 1, flag_at = 0, ntok = 0, flags = 0;
         uint32_t cur = 0;                       // next position, counted from the window's start
         for (uint32_t w0 = 0;; w0 += kHist) {
-            const uint32_t stop = min(n - w0, kCap);    // positions of the window
+            const uint32_t left = n - w0, stop = min(left, kCap);    // positions of the window
             wave_sync();
-            for (uint32_t k = l; k < (kCap + 64) / 4; k += kWave) {
-                uint32_t v[2] = {0, 0};
-                if (w0 / 4 + k < n / 4) __builtin_memcpy(v, __builtin_assume_aligned(rows + 128ull * (w0 / 4 + k), 4), 8);
-                streams[0].data[k] = v[0];
-                streams[1].data[k] = v[1];
-            }
+            for (uint32_t k = l; k < (kCap + 64) / 4; k += kWave)
+                S.data[k] = w0 / 4 + k < n / 4 ? *reinterpret_cast<const uint32_t*>(rows + 128ull * (w0 / 4 + k)) : 0u;
             wave_sync();
             // position 0 is never a candidate, nor one with under 3 bytes left
-            const uint32_t p0 = w0 ? 0u : 1u, left = n - w0;
-            lz_index<kCap>(S, p0, min(stop, left >= kMinLen ? left - (kMinLen - 1) : 0u), sub);
-            while (__ballot(cur < stop)) {
-                const bool on = cur < stop;
-                const uint32_t at = on ? cur : 0;
-                const uint32_t word = lds_u32(bytes + at);
-                const uint32_t h = lz_hash(word);
-                const uint32_t look = on ? min(left - at, kMaxLen) : 0;    // longest match left
-                const uint32_t lo = at >= kHist ? at - kHist + 1 : 0;
-                uint32_t i, e = look >= kMinLen ? ends[h] : 0;
-                if constexpr (LzStream<kCap>::kOld) i = S.first[h];
-                else i = h ? ends[h - 1] : 0;
-                uint32_t key = 0;               // length << 16 | 0xFFFF - position
-                while (__ballot(i < e)) {
-                    const uint32_t best = key >> 16;
-                    const uint32_t q = i + sub < e ? S.slot[i + sub] : 0xFFFFu;
-                    bool live = q < at && q >= lo;
-                    const uint32_t cap = live ? min(at - q, look) : 0;
-                    // a better match agrees on the byte after the best one's
-                    // last, and on the two before it
-                    const uint32_t probe = best >= kMinLen ? best - (kMinLen - 1) : 0;
-                    live = live && cap > best;
-                    const uint32_t qa = live ? q : 0;
-                    const uint32_t x = lds_u32(bytes + qa + probe) ^ lds_u32(bytes + at + probe);
-                    live = live && (x & 0xFFFFFFu) == 0;
-                    uint32_t f = 0;
-                    if (__ballot(live)) {
-                        bool run = live;
-                        while (__ballot(run)) {  // 8 bytes at a time
-                            const uint32_t fa = run ? f : 0, qf = run ? q : 0;
-                            uint64_t a, b;
-                            __builtin_memcpy(&a, bytes + qf + fa, 8);
-                            __builtin_memcpy(&b, bytes + at + fa, 8);
-                            a ^= b;
-                            f = !run ? f : a ? f + ((uint32_t)__builtin_ctzll(a) >> 3) : f + 8;
-                            run = run && !a && f < cap;
+            lz_index<kCap>(S, w0 ? 0u : 1u, min(stop, left >= kMinLen ? left - (kMinLen - 1) : 0u), l);
+            while (cur < stop) {
+                const uint64_t here = lds_u64(S.data, cur);
+                const uint32_t look = min(left - cur, kMaxLen);      // longest match left
+                uint32_t len = 0, from = 0;
+                uint32_t h = lz_hash((uint32_t)here);
+                uint32_t i = uniform(bounds[h]);
+                const uint32_t e = look >= kMinLen ? uniform(bounds[h + 1]) : 0u;
+                if constexpr (LzStream<kCap>::kOld) i = uniform(S.first[h]);
+                for (; i < e; i += kWave) {
+                    const uint32_t q = S.slot[i + l];
+                    const uint32_t qa = q & (kCap - 1);                // slots past the list hold anything
+                    const uint64_t x = lds_u64(S.data, qa) ^ here;
+                    const uint32_t cap = min(cur - q, look);
+                    const bool ok = i + l < e && cur - 1 - q < kHist - 1;   // older, and within reach
+                    uint32_t f = x ? (uint32_t)__builtin_ctzll(x) >> 3 : 8u;
+                    if (__ballot(ok && !x && cap > 8 && cap > len)) {
+                        bool run = ok && !x && cap > 8;
+                        for (uint32_t j = 8; j < kMaxLen; j += 8) {
+                            const uint64_t y = lds_u64(S.data, qa + j) ^ lds_u64(S.data, cur + j);
+                            f = !run ? f : y ? j + ((uint32_t)__builtin_ctzll(y) >> 3) : j + 8;
+                            run = run && !y && cap > j + 8;
+                            if (!__ballot(run)) break;
                         }
-                        f = min(f, cap);
-                        const uint32_t mine = live && f > best && f >= kMinLen ? f << 16 | (0xFFFFu - q) : 0u;
-                        key = max(key, half_max_u32(mine));
+                    }
+                    f = ok ? min(f, cap) : 0u;
+                    // the oldest of the longest: each better one in turn
+                    for (uint64_t m = __ballot(f > max(len, kMinLen - 1)); m; m = __ballot(f > len)) {
+                        const uint32_t lane = (uint32_t)__builtin_ctzll(m);
+                        len = lane_value_at(f, lane);
+                        from = lane_value_at(q, lane);
                     }
                     if constexpr (LzStream<kCap>::kOld) {
                         // a step wholly out of reach stays so for later positions
-                        if (on && i + kHalf <= e && half_ballot(q < lo) == 0xFFFFFFFFu && sub == 0)
-                            S.first[h] = (uint16_t)(i + kHalf);
+                        if (i + kWave <= e && __ballot(q + kHist <= cur) == ~0ull && l == 0) S.first[h] = (uint16_t)(i + kWave);
                     }
-                    i += kHalf;
-                    // younger candidates: none, past the position, or too near to be longer
-                    const uint32_t got = key >> 16;
-                    const uint32_t reach = half_max_u32(q < at ? q : i - kHalf + sub < e ? 0xFFFFu : 0u);
-                    if (got >= look || reach >= at || at - reach <= got) i = e;
+                    if (len >= look || !(__ballot(q < cur) >> (kWave - 1))) break;
                 }
-                if (on) {
-                    const uint32_t len = key >> 16;
-                    if (len == 0) {
-                        if (sub == 0) out[o] = (uint8_t)word;
-                        flags |= 1u << ntok;
-                        o += 1;
-                        cur += 1;
-                    } else {
-                        const uint32_t dist = at - (0xFFFFu - (key & 0xFFFFu));
-                        const uint16_t v = (uint16_t)(dist << kLenBits | (len - kMinLen));
-                        if (sub == 0) __builtin_memcpy(out + o, &v, 2);
-                        o += 2;
-                        cur += len;
-                    }
-                    if (++ntok == 8) {          // the next group's flag byte is reserved at once
-                        if (sub == 0) out[flag_at] = (uint8_t)flags;
-                        flags = 0;
-                        ntok = 0;
-                        flag_at = o++;
-                    }
+                if (len == 0) {
+                    if (l == 0) out[o] = (uint8_t)here;
+                    flags |= 1u << ntok;
+                    o += 1;
+                    cur += 1;
+                } else {
+                    const uint16_t v = (uint16_t)((cur - from) << kLenBits | (len - kMinLen));
+                    if (l == 0) __builtin_memcpy(out + o, &v, 2);
+                    o += 2;
+                    cur += len;
                 }
-                if constexpr (LzStream<kCap>::kOld) wave_sync();    // first[] before its next reader
+                if (++ntok == 8) {              // the next group's flag byte is reserved at once
+                    if (l == 0) out[flag_at] = (uint8_t)flags;
+                    flags = 0;
+                    ntok = 0;
+                    flag_at = o++;
+                }
+                if constexpr (LzStream<kCap>::kOld) wave_sync();        // first[] before its next reader
             }
             if (stop == left) break;
             cur -= kHist;                       // the next window starts kHist positions on
         }
-        if (sub == 0) {
+        if (l == 0) {
             out[flag_at] = (uint8_t)flags;
-            lane_len[lane] = o;
+            lane_len[c * 32 + t] = o;
         }
     }
 }
 
 // Sorted slot of lane t: longer lanes first, equal lengths by higher lane id.
 // Half a wave per chunk.
-constexpr uint32_t kRankThreads = 256, kRankChunks = kRankThreads / kHalf;
+constexpr uint32_t kHalf = 32, kRankThreads = 256, kRankChunks = kRankThreads / kHalf;
 
 __global__ __launch_bounds__(kRankThreads) void lzss_rank_kernel(const uint32_t* __restrict__ lane_len, uint64_t n_chunks,
                                                                  uint64_t* __restrict__ col_len,
@@ -318,7 +280,7 @@ int lzss_compress(const void* in, uint64_t in_bytes, uint64_t chunk, void* work,
     uint32_t* lane_len = reinterpret_cast<uint32_t*>(w + n * 32 * slot);
     uint64_t* chunk_len = reinterpret_cast<uint64_t*>(w + n * 32 * slot + n * chunk * 2);
     const uint32_t lb = (uint32_t)(chunk / 32);
-    const uint64_t units = (n + kXcds - 1) / kXcds * kXcds * kPairs;
+    const uint64_t units = (n + kXcds - 1) / kXcds * kXcds * 32;
     const dim3 grid((uint32_t)(units < (1u << 24) ? units : 1u << 24)), block(kWave);
     auto encode = lb <= 1024 ? lzss_encode_kernel<1024> : lb <= 2048 ? lzss_encode_kernel<2048> : lzss_encode_kernel<4096>;
     hipLaunchKernelGGL(encode, grid, block, 0, s, static_cast<const uint8_t*>(in), n, chunk, slot, w, lane_len);
