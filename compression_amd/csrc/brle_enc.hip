@@ -1,4 +1,4 @@
-// Byte RLE encode for gfx950: one wavefront per chunk.
+// Byte RLE encode for gfx950: one workgroup per chunk.
 //
 // Replaces brle::compress_gpu and its kernels (reference include/brle/
 // brle.h:232-303: one thread runs the byte-at-a-time encoder of :129-230 per
@@ -7,17 +7,27 @@
 //
 // The encoder is a greedy state machine over the chunk's bytes: a pending
 // group is empty, a literal group (up to 128 bytes; a third equal byte in a
-// row ends it and starts a run) or a run (up to 130 equal bytes).  Its
-// decisions change only at the first three bytes of an equal-byte segment,
-// at 128-literal and 130-run limits and at segment ends, so here:
-//   1. per 4 KiB window, every lane compares 64 bytes with their
-//      predecessors and publishes a 64-bit mask of segment starts (LDS);
-//   2. lane 0 walks the window segment by segment (ctz over the masks),
-//      stepping the state machine a constant number of times per segment
-//      and by whole runs otherwise, and appends finished groups
-//      {start, length, run?} to an LDS list;
-//   3. the wave writes the list: a prefix sum over the group sizes places
-//      each group, and each lane writes its group's header and bytes.
+// row ends it and starts a run) or a run (up to 130 equal bytes).  Cut the
+// chunk into segments of equal bytes.  A segment always starts with n = 0..127
+// pending literals (a run ends with its segment), and takes them to
+//   * (n + L) mod 128 if its length L is 1 or 2;
+//   * a value that depends on L alone if L >= 3 and n <= 125: its bytes are
+//     runs of 130 and a rest, which is a run (3 or more) or literals;
+//   * the same after 128 - n literals that fill the group, if n is 126 or 127.
+// So any stretch of segments maps n to n' by {shift; the result for a shifted
+// n below 126, for 126, for 127}, 29 bits, and such maps compose: the state
+// machine is a prefix scan.  Per window of 32 KiB (32 bytes a thread):
+//   1. each thread marks where segments start in its bytes; a scan finds the
+//      segment open before them.  A segment belongs to the thread that sees
+//      the next one start, so no thread looks ahead;
+//   2. it composes its segments' maps, and a scan gives the literals pending
+//      before its first segment;
+//   3. it counts the bytes its segments add, and a scan places them;
+//   4. it writes them to the LDS copy of the output, which the workgroup
+//      stores 16 bytes at a time.  A group's header byte is reserved with its
+//      first literal and written by the segment that ends the group.
+// The scans' latency bounds it (three barriers a window and about 1000 vector
+// instructions a wave), so a workgroup is as wide as the hardware allows.
 // Groups go to a per-chunk slot of the work buffer; a scan kernel turns the
 // chunk sizes into ptr[] and a shift kernel packs the slots into `data`.
 #include "mdz_device.h"
@@ -27,153 +37,270 @@ namespace mdz {
 namespace {
 
 constexpr uint32_t kMinRun = 3, kMaxRun = 130, kMaxLit = 128;
-constexpr uint32_t kWin = 4096;                 // bytes per window: 64 lanes x 64
-constexpr uint32_t kMaxGroups = kWin / 2 + 4;   // a window ends at most this many groups
+constexpr uint32_t kEncThreads = 1024, kEncWaves = kEncThreads / kWave;
+constexpr uint32_t kPer = 32;                   // bytes per thread and window
+constexpr uint32_t kWin = kEncThreads * kPer;
+constexpr uint32_t kStage = kWin + kWin / 32;   // staged output bytes of a window
 
 struct EncLds {
-    uint64_t starts[kWave];                     // bit j of word l: byte 64 l + j starts a segment
-    uint32_t g_start[kMaxGroups];               // chunk offset of the group's first byte
-    uint32_t g_len[kMaxGroups];                 // bytes << 1 | run
+    alignas(16) uint32_t in[kWin / 4];
+    alignas(16) uint32_t out[kStage / 4 + 8];
+    uint32_t part[3][kEncWaves];
 };
 
-enum : uint32_t { kEmpty = 0, kLit = 1, kRun = 2 };
+// Pending literals after a segment of L >= 3 bytes that starts as runs.
+MDZ_DEV uint32_t rest_of(uint32_t L) {
+    const uint32_t r = L % kMaxRun;
+    return r < kMinRun ? r : 0;
+}
+// Output bytes of that segment: whole runs, then a run or a header and literals.
+MDZ_DEV uint32_t run_bytes(uint32_t L) {
+    const uint32_t r = L % kMaxRun;
+    return 2 * (L / kMaxRun) + (r >= kMinRun ? 2 : r ? r + 1 : 0);
+}
 
-struct Machine {
-    uint32_t mode = kEmpty, n = 0, tail = 0, start = 0, groups = 0;
+// A map of pending literals: bits 0..6 shift, then (bit 31 set) the results
+// for a shifted count below 126, of 126 and of 127.
+constexpr uint32_t kReset = 1u << 31;
+MDZ_DEV uint32_t map_apply(uint32_t f, uint32_t n) {
+    const uint32_t t = (n + f) & 127;
+    const uint32_t r = f >> (t < 126 ? 7 : t == 126 ? 14 : 21);
+    return f & kReset ? r & 127 : t;
+}
+MDZ_DEV uint32_t map_then(uint32_t f, uint32_t g) {      // f, then g
+    const uint32_t shifted = (g & ~127u) | ((f + g) & 127);
+    const uint32_t through = kReset | (f & 127) | map_apply(g, (f >> 7) & 127) << 7 |
+                             map_apply(g, (f >> 14) & 127) << 14 | map_apply(g, (f >> 21) & 127) << 21;
+    return f & kReset ? through : shifted;
+}
+MDZ_DEV uint32_t map_of(uint32_t L) {
+    if (L < kMinRun) return L;
+    const uint32_t b = L - 2 >= kMinRun ? rest_of(L - 2) : L - 2, c = L - 1 >= kMinRun ? rest_of(L - 1) : L - 1;
+    return kReset | rest_of(L) << 7 | b << 14 | c << 21;
+}
+MDZ_DEV uint32_t wave_incl_maps(uint32_t v) {
+    v = map_then(dpp_src<0x111, 0xf, 0u>(v), v);          // the identity is 0
+    v = map_then(dpp_src<0x112, 0xf, 0u>(v), v);
+    v = map_then(dpp_src<0x114, 0xf, 0u>(v), v);
+    v = map_then(dpp_src<0x118, 0xf, 0u>(v), v);
+    v = map_then(dpp_src<0x142, 0xa, 0u>(v), v);
+    v = map_then(dpp_src<0x143, 0xc, 0u>(v), v);
+    return v;
+}
+MDZ_DEV uint32_t wave_incl_max_u32(uint32_t v) {
+    v = max(v, dpp_src<0x111, 0xf, 0u>(v));
+    v = max(v, dpp_src<0x112, 0xf, 0u>(v));
+    v = max(v, dpp_src<0x114, 0xf, 0u>(v));
+    v = max(v, dpp_src<0x118, 0xf, 0u>(v));
+    v = max(v, dpp_src<0x142, 0xa, 0u>(v));
+    v = max(v, dpp_src<0x143, 0xc, 0u>(v));
+    return v;
+}
+// The value of the lane below; `first` in lane 0.
+MDZ_DEV uint32_t from_below(uint32_t v, uint32_t first) {
+    const uint32_t r = (uint32_t)__shfl_up((int)v, 1, kWave);
+    return lane_id() ? r : first;
+}
 
-    MDZ_DEV void emit(EncLds& S, uint32_t at, uint32_t len, uint32_t run) {
-        S.g_start[groups] = at;
-        S.g_len[groups] = len << 1 | run;
-        ++groups;
+// Output bytes of a segment of L bytes after n pending literals; n moves on.
+MDZ_DEV uint32_t count_segment(uint32_t& n, uint32_t L) {
+    uint32_t bytes = 0;
+    if (L >= kMinRun && n >= 126) {             // the group fills up first
+        bytes = kMaxLit - n;
+        L -= bytes;
+        n = 0;
     }
-    // Bytes [p, q) are equal; `fresh` != 0: byte p differs from byte p - 1.
-    MDZ_DEV void feed(EncLds& S, uint32_t p, uint32_t q, uint32_t fresh) {
-        if (fresh && mode == kRun) {            // a run ends where the byte changes
-            emit(S, start, n, 1);
-            mode = kEmpty;
+    if (L >= kMinRun) {
+        bytes += run_bytes(L);
+        n = rest_of(L);
+    } else {
+        bytes += L + (n == 0 && L ? 1u : 0u) + (n + L > kMaxLit ? 1u : 0u);
+        n = (n + L) & (kMaxLit - 1);
+    }
+    return bytes;
+}
+
+// Writes that segment's bytes of value v at offset o (relative to the output
+// so far) through put(offset, byte); returns the offset after them.
+template <class Put>
+MDZ_DEV int32_t write_segment(Put put, int32_t o, uint32_t& n, uint32_t L, uint32_t v) {
+    auto literals = [&](uint32_t k) {
+        for (; k; --k) {
+            if (n == 0) ++o;                    // the header's place
+            put(o++, v);
+            if (++n == kMaxLit) {
+                put(o - 1 - (int32_t)kMaxLit, kMaxLit + 127);
+                n = 0;
+            }
         }
-        uint32_t same = fresh ? 0u : 1u;
-        while (p < q) {
-            if (mode == kEmpty) {
-                mode = kLit;
-                start = p;
-                n = 1;
-                tail = 1;
-                ++p;
-                same = 1;
-                continue;
-            }
-            if (mode == kRun) {
-                const uint32_t take = min(q - p, kMaxRun - n);
-                n += take;
-                p += take;
-                if (n == kMaxRun) {
-                    emit(S, start, n, 1);
-                    mode = kEmpty;
-                }
-                continue;
-            }
-            tail = same ? tail + 1 : 1;         // literal group: one byte
-            if (tail == kMinRun) {
-                if (n + 1 != kMinRun) {          // the group's last two bytes join the run
-                    emit(S, start, n - (kMinRun - 1), 0);
-                    start = p - (kMinRun - 1);
-                }
-                mode = kRun;
-                n = kMinRun;
-            } else if (++n == kMaxLit) {
-                emit(S, start, n, 0);
-                mode = kEmpty;
-            }
-            ++p;
-            same = 1;
-        }
+    };
+    if (L >= kMinRun && n >= 126) {
+        const uint32_t fill = kMaxLit - n;
+        literals(fill);
+        L -= fill;
     }
-    MDZ_DEV void finish(EncLds& S) {
-        if (mode != kEmpty) emit(S, start, n, mode == kRun ? 1u : 0u);
-        mode = kEmpty;
+    if (L < kMinRun) {
+        literals(L);
+        return o;
     }
-};
+    if (n) put(o - 1 - (int32_t)n, n + 127);
+    n = 0;
+    for (; L >= kMinRun; L -= min(L, kMaxRun)) {
+        put(o, min(L, kMaxRun) - kMinRun);
+        put(o + 1, v);
+        o += 2;
+    }
+    literals(L);
+    return o;
+}
 
-__global__ __launch_bounds__(kWave) void brle_encode_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes,
-                                                            uint64_t chunk, uint64_t slot,
-                                                            uint8_t* __restrict__ work,
-                                                            uint64_t* __restrict__ sizes) {
+// Exclusive scan over the workgroup through part[16]: `incl` is the wave's
+// inclusive scan, `carry` comes before the workgroup's first thread and takes
+// in its last.  One barrier.
+template <class Then>
+MDZ_DEV uint32_t block_scan(uint32_t* part, uint32_t incl, uint32_t& carry, Then then) {
+    const uint32_t wave = threadIdx.x / kWave;
+    if (lane_id() == kWave - 1) part[wave] = incl;
+    __syncthreads();
+    uint32_t before = carry, all = carry;
+    for (uint32_t w = 0; w < kEncWaves; ++w) {
+        all = then(all, part[w]);
+        if (w + 1 == wave) before = all;
+    }
+    carry = all;
+    return then(before, from_below(incl, 0));
+}
+
+__global__ __launch_bounds__(kEncThreads) void brle_encode_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes,
+                                                                  uint64_t chunk, uint64_t slot,
+                                                                  uint8_t* __restrict__ work,
+                                                                  uint64_t* __restrict__ sizes) {
     __shared__ EncLds S;
-    const uint32_t l = lane_id();
+    const uint32_t t = threadIdx.x;
     const uint64_t c = blockIdx.x;
     const uint64_t base = c * chunk;
     const uint32_t len = (uint32_t)min(chunk, in_bytes - base);
     const uint8_t* src = in + base;
     uint8_t* out = work + c * slot;
-    Machine m;                                  // lane 0's
-    uint64_t written = 0;
-    for (uint32_t w0 = 0; w0 < len; w0 += kWin) {
-        const uint32_t wl = min(kWin, len - w0);
-        // 1. segment starts of this window: the lane's 64 bytes, loaded
-        //    without branches (positions past the chunk read its last byte
-        //    and are masked off)
-        const uint32_t end = w0 + wl;
-        const uint32_t lo = w0 + 64 * l;
-        uint32_t prev = lo == 0 ? 0x100u : src[min(lo, len) - 1];
-        uint64_t mask = 0;
+    const uint8_t* in8 = reinterpret_cast<const uint8_t*>(S.in);
+    uint8_t* out8 = reinterpret_cast<uint8_t*>(S.out);
+    const uint32_t skew = (uint32_t)((uintptr_t)src & 3);
+    uint32_t open = 0;                          // start of the segment open before the window
+    uint32_t state = 0;                         // map of the segments before the window: pending literals
+    uint32_t last = 0x100;                      // the byte before the window
+    uint64_t done = 0;                          // output bytes before the window
+    uint64_t staged = 0;                        // the output from here on is in LDS, not yet in `out`
+    for (uint32_t w0 = 0; w0 < len; w0 += min(kWin, len - w0)) {
+        // 1. the thread's bytes: to LDS, and where they differ from the byte before
+        const uint32_t wl = min(kWin, len - w0), at = kPer * t;
+        uint32_t v[kPer / 4];
+        if (at + kPer <= wl && ((uintptr_t)src & 15) == 0) {
+            const uint4* p = reinterpret_cast<const uint4*>(src + w0 + at);
 #pragma unroll
-        for (uint32_t j = 0; j < 64; ++j) {
-            const uint32_t v = src[min(lo + j, len - 1)];
-            if (v != prev) mask |= 1ull << j;
-            prev = v;
-        }
-        S.starts[l] = lo >= end ? 0 : end - lo >= 64 ? mask : mask & ((1ull << (end - lo)) - 1);
-        wave_sync();
-        // 2. the state machine, one equal-byte piece at a time: a piece ends
-        //    at the next set bit of the masks, or at the window's end
-        if (l == 0) {
-            m.groups = 0;
-            uint32_t p = w0;
-            const uint32_t nw = (wl + 63) / 64;
-            uint32_t fresh = (uint32_t)(S.starts[0] & 1);
-            for (uint32_t k = 0; k < nw; ++k) {
-                uint64_t bits = S.starts[k];
-                if (k == 0) bits &= ~1ull;               // byte w0 opens the first piece
-                while (bits) {
-                    const uint32_t q = w0 + 64 * k + (uint32_t)__builtin_ctzll(bits);
-                    m.feed(S, p, q, fresh);
-                    p = q;
-                    fresh = 1;
-                    bits &= bits - 1;
-                }
+            for (uint32_t i = 0; i < kPer / 16; ++i) {
+                const uint4 q = p[i];
+                v[4 * i] = q.x, v[4 * i + 1] = q.y, v[4 * i + 2] = q.z, v[4 * i + 3] = q.w;
             }
-            m.feed(S, p, end, fresh);
-            if (end == len) m.finish(S);
-        }
-        wave_sync();
-        // 3. write the finished groups in order
-        const uint32_t ng = __builtin_amdgcn_readfirstlane(m.groups);
-        for (uint32_t g0 = 0; g0 < ng; g0 += kWave) {
-            const uint32_t g = g0 + l;
-            uint32_t at = 0, gl = 0, sz = 0;
-            if (g < ng) {
-                at = S.g_start[g];
-                gl = S.g_len[g];
-                sz = (gl & 1) ? 2 : 1 + (gl >> 1);
+        } else if (w0 + at >= skew && w0 + at + kPer + 4 <= len) {
+            // whole dwords around the bytes, shifted together
+            const uint32_t* p = reinterpret_cast<const uint32_t*>(src + w0 + at - skew);
+            uint32_t lo = p[0];
+#pragma unroll
+            for (uint32_t i = 0; i < kPer / 4; ++i) {
+                const uint32_t hi = p[i + 1];
+                v[i] = alignbyte(hi, lo, skew);
+                lo = hi;
             }
-            const uint32_t incl = wave_incl_scan_u32(sz);
-            uint8_t* o = out + written + (incl - sz);
-            if (g < ng) {
-                const uint32_t n = gl >> 1;
-                if (gl & 1) {
-                    o[0] = (uint8_t)(n - kMinRun);
-                    o[1] = src[at];
+        } else {                                // the chunk's first or last bytes
+#pragma unroll
+            for (uint32_t i = 0; i < kPer; ++i) {
+                const uint32_t b = at + i < wl ? src[w0 + at + i] : 0u;
+                v[i / 4] = i & 3 ? v[i / 4] | b << (8 * (i & 3)) : b;
+            }
+        }
+#pragma unroll
+        for (uint32_t i = 0; i < kPer / 4; ++i) S.in[at / 4 + i] = v[i];
+        __syncthreads();
+        uint32_t before = t ? in8[at - 1] : last, mask = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kPer / 4; ++i) {
+            const uint32_t x = v[i] ^ (v[i] << 8 | (before & 0xFFu));
+            const uint32_t nz = ((((x & 0x7F7F7F7Fu) + 0x7F7F7F7Fu) | x) >> 7) & 0x01010101u;
+            mask |= ((nz * 0x10204080u) >> 28) << (4 * i);
+            before = v[i] >> 24;
+        }
+        if (w0 + t == 0) mask |= 1;             // the chunk's first byte opens a segment
+        mask = at >= wl ? 0 : wl - at >= kPer ? mask : mask & ((1u << (wl - at)) - 1);
+        const uint32_t newest = mask ? w0 + at + 31 - __builtin_clz(mask) : 0;
+        const uint32_t prev0 = block_scan(S.part[0], wave_incl_max_u32(newest), open,
+                                          [](uint32_t a, uint32_t b) { return max(a, b); });
+        // the segments that end in these bytes (position 0 ends none)
+        const uint32_t ends = w0 + t == 0 ? mask & ~1u : mask;
+        auto each = [&](auto fn) {
+            uint32_t prev = prev0;
+            for (uint32_t m = ends; m; m &= m - 1) {
+                const uint32_t b = (uint32_t)__builtin_ctz(m), p = w0 + at + b;
+                fn(p - prev, at + b);
+                prev = p;
+            }
+        };
+        // 2. literals pending before the thread's first segment
+        uint32_t map = 0;
+        each([&](uint32_t L, uint32_t) { map = map_then(map, map_of(L)); });
+        uint32_t n = map_apply(block_scan(S.part[1], wave_incl_maps(map), state, map_then), 0);
+        // 3. where its bytes go
+        uint32_t bytes = 0, n3 = n;
+        each([&](uint32_t L, uint32_t) { bytes += count_segment(n3, L); });
+        uint32_t total = 0;
+        const uint32_t off = block_scan(S.part[2], wave_incl_scan_u32(bytes), total,
+                                        [](uint32_t a, uint32_t b) { return a + b; });
+        // 4. write them.  LDS byte i holds output byte (staged & ~15) + i; what
+        // does not fit there (long runs), and headers stored before, go straight out
+        const uint64_t stage0 = staged & ~15ull;
+        const bool fits = done + total - stage0 <= kStage;
+        const int32_t held = (int32_t)(int64_t)(staged - done), shift = (int32_t)(int64_t)(done - stage0);
+        if (!fits) {
+            for (uint64_t i = staged + t; i < done; i += kEncThreads) out[i] = out8[i - stage0];
+            __syncthreads();
+        }
+        auto put = [&](int32_t o, uint32_t b) {
+            if (fits && o >= held) out8[o + shift] = (uint8_t)b;
+            else out[(int64_t)done + o] = (uint8_t)b;
+        };
+        int32_t o = (int32_t)off;
+        each([&](uint32_t L, uint32_t p) { o = write_segment(put, o, n, L, p ? in8[p - 1] : last); });
+        last = in8[wl - 1];
+        __syncthreads();
+        done += total;
+        if (fits) {                             // store whole 16-byte units, keep the rest
+            const uint64_t whole = w0 + wl == len ? done : max(done & ~15ull, staged);
+            for (uint64_t u = stage0 + 16 * t; u < whole; u += 16 * kEncThreads) {
+                const uint32_t i = (uint32_t)(u - stage0);
+                if (u >= staged && u + 16 <= whole) {
+                    *reinterpret_cast<uint4*>(out + u) = *reinterpret_cast<const uint4*>(out8 + i);
                 } else {
-                    o[0] = (uint8_t)(n + 127);
-                    for (uint32_t i = 0; i < n; ++i) o[1 + i] = src[at + i];
+                    for (uint32_t k = 0; k < 16; ++k)
+                        if (u + k >= staged && u + k < whole) out[u + k] = out8[i + k];
                 }
             }
-            written += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
+            const uint32_t rest = (uint32_t)(done - whole);       // under 16 bytes
+            const uint32_t keep = t < rest ? out8[(uint32_t)(whole - stage0) + t] : 0u;
+            __syncthreads();
+            if (t < rest) out8[(uint32_t)(whole & 15) + t] = (uint8_t)keep;
+            staged = whole;
+        } else {
+            staged = done;
         }
-        wave_sync();
     }
-    if (l == 0) sizes[c] = written;
+    // the last segment, and the literals still pending
+    __syncthreads();
+    uint32_t n = map_apply(state, 0);
+    auto put = [&](int32_t o, uint32_t b) { out[(int64_t)done + o] = (uint8_t)b; };
+    if (t == 0) {
+        const int32_t o = write_segment(put, 0, n, len - open, last);
+        if (n) put(o - 1 - (int32_t)n, n + 127);
+        sizes[c] = done + (uint32_t)o;
+    }
 }
 
 // ptr[0] = 0, ptr[c + 1] = ptr[c] + sizes[c]: one workgroup, each thread
@@ -250,7 +377,7 @@ int brle_compress(const void* in, uint64_t in_bytes, uint64_t chunk, void* work,
     if (n > (1ull << 24)) return MDZ_ERR_INVALID;     // grid sizes stay below 2^32 threads
     const uint64_t slot = (wb - 8 * n) / n;
     uint64_t* sizes = reinterpret_cast<uint64_t*>(static_cast<uint8_t*>(work) + n * slot);
-    hipLaunchKernelGGL(brle_encode_kernel, dim3((uint32_t)n), dim3(kWave), 0, s,
+    hipLaunchKernelGGL(brle_encode_kernel, dim3((uint32_t)n), dim3(kEncThreads), 0, s,
                        static_cast<const uint8_t*>(in), in_bytes, chunk, slot, static_cast<uint8_t*>(work), sizes);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return record_hip(e, "brle_encode_kernel launch");

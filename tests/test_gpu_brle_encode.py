@@ -59,3 +59,37 @@ def test_reference_container_and_roundtrip(gpu):
     blob = brle.compress_gpu(data.tobytes())
     assert blob == host.brle_encode(data, 262144).to_bytes()
     assert brle.decompress_gpu(blob) == data.tobytes()
+
+
+def _segments(size, lengths, seed):
+    """Equal-byte segments of the given lengths in random order, neighbours different."""
+    rng = np.random.default_rng(seed)
+    k = rng.choice(lengths, size // max(1, sum(lengths) // len(lengths)) + 2 * len(lengths) + 64)
+    k = np.minimum(k, size)
+    v = np.cumsum(1 + rng.integers(0, 255, k.size)) % 256
+    out = np.repeat(v.astype(np.uint8), k)
+    return np.resize(out, size)
+
+
+# segment lengths that meet the 128-literal and 130-run limits from every
+# phase; chunks around the 32 KiB window, of odd sizes (so chunks start at any
+# byte) and with runs longer than a window's staged output
+@pytest.mark.parametrize("lengths", [[1], [1, 2], [1, 2, 3], [1, 2, 125, 126, 127, 128, 129],
+                                     [1, 3, 129, 130, 131, 132, 133, 259, 260, 261, 262, 263],
+                                     [1, 2, 40_000], [1, 5_000_000]])
+@pytest.mark.parametrize("chunk", [1, 127, 1000, 32767, 32768, 32769, 65541, 262144, 9_000_000])
+def test_segment_lengths(gpu, lengths, chunk):
+    from compression_amd import brle
+    from compression_amd._lib import DeviceBuffer
+    size = min(300 * chunk, 200_000 if chunk < 200_000 else 2 * chunk + 12345)
+    data = _segments(size, lengths, chunk + len(lengths))
+    for skip in (0, 1, 6):                     # the input's own alignment
+        n, wb, cap = brle.compress_bound(size - skip, chunk)
+        src = DeviceBuffer.from_array(data)
+        work, dst, ptr = DeviceBuffer(wb), DeviceBuffer(cap), DeviceBuffer(8 * (n + 1))
+        print(f"brle encode lengths={lengths} chunk={chunk} skip={skip} n={n}", flush=True)
+        brle.compress(src.ptr + skip, size - skip, dst, ptr, work, chunk_bytes=chunk)
+        ref = host.brle_encode(data[skip:], chunk)
+        got = ptr.download(8 * (n + 1)).view(np.uint64)
+        assert np.array_equal(got, ref.ptr)
+        assert dst.download(int(got[-1])).tobytes() == ref.data.tobytes()
