@@ -10,6 +10,40 @@
 namespace mdz {
 namespace {
 
+// A wave (one workgroup) per lane stream.  A chunk's 32 streams read the same
+// input lines: units are numbered so that they run on one XCD (workgroups go
+// to the XCDs in turn), whose L2 then reads each line once.
+constexpr uint32_t kXcds = 8;
+
+__host__ __device__ inline uint64_t lane_units(uint64_t n_chunks) {
+    return (n_chunks + kXcds - 1) / kXcds * kXcds * 32;
+}
+MDZ_DEV bool lane_of_unit(uint64_t unit, uint64_t n_chunks, uint64_t& c, uint32_t& t) {
+    t = (uint32_t)(unit / kXcds) % 32;
+    c = unit / (kXcds * 32) * kXcds + unit % kXcds;
+    return c < n_chunks;
+}
+inline dim3 lane_grid(uint64_t n_chunks) {       // the kernels stride over the units beyond it
+    const uint64_t u = lane_units(n_chunks);
+    return dim3((uint32_t)(u < (1u << 24) ? u : 1u << 24));
+}
+
+// chunk_len[c]: the chunk's lanes rounded up to words, their sum to 128
+// bytes.  Half a wave per chunk.
+constexpr uint32_t kSizeThreads = 256, kSizeChunks = kSizeThreads / 32;
+
+__global__ __launch_bounds__(kSizeThreads) void lanes_size_kernel(const uint64_t* __restrict__ col_len, uint64_t n,
+                                                                  uint64_t* __restrict__ chunk_len) {
+    const uint64_t c = (uint64_t)blockIdx.x * kSizeChunks + threadIdx.x / 32;
+    const uint32_t words = c < n ? (uint32_t)((col_len[c * 32 + threadIdx.x % 32] + 3) / 4) : 0u;
+    const uint32_t incl = wave_incl_scan_u32(words);
+    const uint32_t low = (uint32_t)__builtin_amdgcn_readlane((int)incl, 31);
+    if (c < n && threadIdx.x % 32 == 31) {
+        const uint32_t total = lane_id() < 32 ? incl : incl - low;
+        chunk_len[c] = ((uint64_t)total * 4 + 127) / 128 * 128;
+    }
+}
+
 constexpr uint32_t kScanThreads = 1024;
 
 __global__ __launch_bounds__(kScanThreads) void lanes_scan_kernel(const uint64_t* __restrict__ sizes, uint64_t n,

@@ -37,7 +37,6 @@ namespace {
 
 constexpr uint32_t kHist = 2048, kMinLen = 3, kMaxLen = 34, kLenBits = 5;
 constexpr uint32_t kHashBits = 9, kBuckets = 1u << kHashBits;
-constexpr uint32_t kXcds = 8;
 
 // One lane stream's window: kCap positions and the bytes a match at the last
 // of them can reach.
@@ -137,13 +136,10 @@ __global__ __launch_bounds__(kWave) void lzss_encode_kernel(const uint8_t* __res
     const uint32_t l = lane_id();
     const uint16_t* bounds = reinterpret_cast<const uint16_t*>(S.bound);
     const uint32_t n = (uint32_t)(chunk / 32);
-    // A chunk's 32 lanes read the same 128-byte rows: they run on one XCD
-    // (workgroups go to the XCDs in turn), so its L2 reads each row once.
-    const uint64_t units = (n_chunks + kXcds - 1) / kXcds * kXcds * 32;
-    for (uint64_t unit = blockIdx.x; unit < units; unit += gridDim.x) {
-        const uint32_t t = (uint32_t)(unit / kXcds) % 32;
-        const uint64_t c = unit / (kXcds * 32) * kXcds + unit % kXcds;
-        if (c >= n_chunks) continue;
+    for (uint64_t unit = blockIdx.x; unit < lane_units(n_chunks); unit += gridDim.x) {
+        uint64_t c;
+        uint32_t t;
+        if (!lane_of_unit(unit, n_chunks, c, t)) continue;
         const uint8_t* rows = in + c * chunk + 4 * t;
         uint8_t* out = work + (c * 32 + t) * lane_slot;
         uint32_t o = 1, flag_at = 0, ntok = 0, flags = 0;
@@ -280,8 +276,7 @@ int lzss_compress(const void* in, uint64_t in_bytes, uint64_t chunk, void* work,
     uint32_t* lane_len = reinterpret_cast<uint32_t*>(w + n * 32 * slot);
     uint64_t* chunk_len = reinterpret_cast<uint64_t*>(w + n * 32 * slot + n * chunk * 2);
     const uint32_t lb = (uint32_t)(chunk / 32);
-    const uint64_t units = (n + kXcds - 1) / kXcds * kXcds * 32;
-    const dim3 grid((uint32_t)(units < (1u << 24) ? units : 1u << 24)), block(kWave);
+    const dim3 grid = lane_grid(n), block(kWave);
     auto encode = lb <= 1024 ? lzss_encode_kernel<1024> : lb <= 2048 ? lzss_encode_kernel<2048> : lzss_encode_kernel<4096>;
     hipLaunchKernelGGL(encode, grid, block, 0, s, static_cast<const uint8_t*>(in), n, chunk, slot, w, lane_len);
     hipError_t e = hipGetLastError();

@@ -63,3 +63,57 @@ def test_roundtrip_through_decoder(gpu):
     rlev2.decompress(lanes, dst, raw.size, st)
     assert (st.download(4 * n).view(np.int32) == 0).all()
     assert dst.download(raw.size).tobytes() == raw.tobytes()
+
+
+def _shapes(n, seed):
+    """Columns that meet every sub-mode at its limits: runs around 3, 10 and
+    128 values, sorted and wrapping deltas, narrow values with zeros, patches."""
+    rng = np.random.default_rng(seed)
+    k = rng.choice([1, 2, 3, 4, 9, 10, 11, 12, 126, 127, 128, 129, 130, 131, 255, 256, 257, 300], n)
+    v = rng.integers(0, 2**40, n).astype(np.uint64)
+    v[::3] = 0
+    steps = np.cumsum(rng.integers(0, 1000, n)).astype(np.uint64)
+    seg, have = [], 0
+    while have < n:
+        m = int(rng.integers(1, 200))
+        w = int(rng.integers(1, 63))
+        s = rng.integers(0, 2**w, m)
+        kind = rng.integers(0, 5)
+        if kind == 0:
+            s = s[0] // 2 + np.arange(m) * int(rng.integers(0, 100))
+        elif kind == 1:
+            s = np.where(rng.random(m) < 0.05, rng.integers(2**40, 2**62, m), s % 2**16)
+        elif kind == 2:
+            s = np.sort(s)[::int(rng.choice([1, -1]))]
+        elif kind == 3:
+            s = rng.integers(0, 2, m) * int(rng.integers(1, 300))
+        seg.append(np.asarray(s, np.int64).view(np.uint64))
+        have += m
+    return {"runs": np.repeat(v, k)[:n], "up": steps, "down": np.uint64(1 << 62) - steps,
+            "wrap": np.cumsum(rng.integers(0, 2**62, n).astype(np.uint64)), "zeros": np.zeros(n, np.uint64),
+            "narrow": rng.integers(0, 130, n).astype(np.uint64), "mix": np.concatenate(seg)[:n]}
+
+
+# lanes of 1 value to several LDS windows (512 values of 8 bytes, 1024 of less)
+@pytest.mark.parametrize("dtype", [np.uint64, np.uint32, np.uint16, np.uint8])
+@pytest.mark.parametrize("lane_values,ru", [(1, 1), (3, 3), (40, 4), (128, 16), (512, 512), (513, 27), (1300, 13),
+                                            (4096, 64)])
+def test_group_limits(gpu, dtype, lane_values, ru):
+    from compression_amd import rlev2
+    from compression_amd._lib import DeviceBuffer
+    eb = np.dtype(dtype).itemsize
+    chunk, nvals = 32 * lane_values * eb, min(32 * lane_values * 2 - 5, 200_000)
+    for name, x in _shapes(max(nvals, 64), lane_values + eb).items():
+        data = (x[:nvals] >> np.uint64(0 if eb == 8 else 5)).astype(dtype)
+        raw = data.view(np.uint8)
+        n, wb, cap = rlev2.compress_bound(raw.size, chunk, eb, ru)
+        src, work, pay, pb = DeviceBuffer.from_array(raw), DeviceBuffer(wb), DeviceBuffer(cap), DeviceBuffer(8)
+        col, off = DeviceBuffer(256 * n), DeviceBuffer(8 * (n + 1))
+        print(f"rlev2 encode {name} {eb} bytes, {lane_values} lane values, ru={ru} n={n}", flush=True)
+        rlev2.compress(src, raw.size, chunk, eb, ru, work, pay, col, off, pb)
+        ref = host.rlev2_encode(data, chunk, ru)
+        assert np.array_equal(off.download(8 * (n + 1)).view(np.uint64), ref.blk_off), name
+        assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len), name
+        nbytes = int(pb.download(8).view(np.uint64)[0])
+        assert nbytes == ref.payload_bytes, name
+        assert pay.download(nbytes).tobytes() == ref.payload[:nbytes].tobytes(), name
