@@ -60,3 +60,40 @@ def test_host_form_roundtrip(gpu, tmp_path, monkeypatch):
     col = np.fromfile("input_data/rle_v1_col_len.bin", np.uint64)
     off = np.fromfile("input_data/rle_v1_blk_offset.bin", np.uint64)
     assert rle_v1.decompress_gpu(blob, 128, 131072, 4, col, off) == data.tobytes()
+
+
+# lane streams around the encoder's 64-value windows, with runs and literal
+# groups that reach, meet and pass their limits (129 and 127) across windows
+@pytest.mark.parametrize("dtype", [np.uint32, np.uint64, np.uint16, np.uint8])
+@pytest.mark.parametrize("lane_values,line_values", [(2, 1), (3, 3), (61, 61), (62, 2), (63, 1), (64, 8), (126, 6),
+                                                     (130, 10), (2000, 40)])
+def test_token_limits(gpu, dtype, lane_values, line_values):
+    from compression_amd import rle_v1
+    from compression_amd._lib import DeviceBuffer
+    eb = np.dtype(dtype).itemsize
+    chunk, nvals = 32 * lane_values * eb, min(32 * lane_values * 3 - 3, 200_000)
+    rng = np.random.default_rng(lane_values + eb)
+    seg, have = [], 0
+    while have < nvals:
+        m = int(rng.choice([1, 2, 3, 4, 63, 64, 65, 126, 127, 128, 129, 130, 131, 257, 258, 259]))
+        w = int(rng.integers(1, 62))
+        s = rng.integers(0, 2**w, m)
+        kind = rng.integers(0, 3)
+        if kind:
+            s = s[0] + np.arange(m) * (int(rng.integers(-130, 130)) if kind == 1 else 0)
+        seg.append(np.asarray(s, np.int64).view(np.uint64))
+        have += m
+    for name, x in {"mix": np.concatenate(seg)[:nvals], "run": np.arange(nvals, dtype=np.uint64) * np.uint64(3),
+                    "literals": rng.integers(0, 2**62, nvals).astype(np.uint64)}.items():
+        data = x.astype(dtype)
+        raw = data.view(np.uint8)
+        n, wb, cap = rle_v1.compress_bound(raw.size, chunk, eb, line_values * eb)
+        src, work, pay = DeviceBuffer.from_array(raw), DeviceBuffer(wb), DeviceBuffer(cap)
+        col, off = DeviceBuffer(256 * n), DeviceBuffer(8 * (n + 1))
+        print(f"rlev1 encode {name} {eb} bytes, {lane_values} lane values n={n}", flush=True)
+        rle_v1.compress(src, raw.size, chunk, eb, line_values * eb, work, pay, col, off)
+        ref = host.rlev1_encode(data, chunk, line_values * eb)
+        got = off.download(8 * (n + 1)).view(np.uint64)
+        assert np.array_equal(got, ref.blk_off), name
+        assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len), name
+        assert pay.download(int(got[-1])).tobytes() == ref.payload[:int(got[-1])].tobytes(), name
