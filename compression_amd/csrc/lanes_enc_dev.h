@@ -69,14 +69,19 @@ __global__ __launch_bounds__(kScanThreads) void lanes_scan_kernel(const uint64_t
     }
 }
 
-constexpr uint32_t kIlvThreads = 256;
+// Interleave.  Word r of slot t lands at base(r) + #{t' < t : words_t' > r},
+// with base(r) = sum_t' min(words_t', r).  Per tile of 128 rounds base and the
+// mask of slots still holding words are computed once per round, the slots'
+// words are read along the streams (256 bytes a wave and load, 16 loads in
+// flight), put in order in LDS (one word of padding per 32, or the 64 words of
+// a load would share two banks) and stored along the chunk.  Few chunks are
+// split over `parts` workgroups, tile by tile, so that the chip is full.
+// 64 MiB of 4-byte RLE v1 values (512 chunks): 113 us with one workgroup per
+// chunk scattering words straight to memory.
+constexpr uint32_t kIlvThreads = 256, kIlvWaves = kIlvThreads / kWave;
+constexpr uint32_t kRoundTile = 2 * kWave;
+constexpr uint32_t kIlvGroups = 2048;            // workgroups that fill the chip: 8 a CU
 
-constexpr uint32_t kRoundTile = 1024;
-
-// Word r of slot t lands at base(r) + #{t' < t : words_t' > r}, with
-// base(r) = sum_t' min(words_t', r).  Per tile of rounds, base and the mask of
-// slots still holding words are computed once per round (LDS); each word then
-// costs a popcount.
 __global__ __launch_bounds__(kIlvThreads) void lanes_interleave_kernel(const uint8_t* __restrict__ work,
                                                                        uint64_t lane_slot,
                                                                        const uint64_t* __restrict__ col_len,
@@ -84,11 +89,16 @@ __global__ __launch_bounds__(kIlvThreads) void lanes_interleave_kernel(const uin
                                                                        const uint64_t* __restrict__ chunk_len,
                                                                        const uint8_t* __restrict__ lane_map,
                                                                        uint8_t* __restrict__ payload) {
-    __shared__ uint32_t words[32];
-    __shared__ uint32_t rbase[kRoundTile], rmask[kRoundTile];
-    const uint32_t tid = threadIdx.x;
+    constexpr uint32_t kSlots = 32 / kIlvWaves;   // slots a wave reads
+    __shared__ uint32_t words[32], bytes[32];
+    __shared__ uint32_t rbase[kRoundTile + 1], rmask[kRoundTile];
+    __shared__ uint32_t tile[kRoundTile * 33];
+    const uint32_t tid = threadIdx.x, l = lane_id(), t0 = tid / kWave * kSlots;
     const uint64_t c = blockIdx.x;
-    if (tid < 32) words[tid] = (uint32_t)((col_len[c * 32 + tid] + 3) / 4);
+    if (tid < 32) {
+        bytes[tid] = (uint32_t)col_len[c * 32 + tid];
+        words[tid] = (bytes[tid] + 3) / 4;
+    }
     __syncthreads();
     uint32_t* dst = reinterpret_cast<uint32_t*>(payload + blk_off[c]);   // blk_off is a multiple of 128
     uint32_t total = 0, maxw = 0;
@@ -96,36 +106,59 @@ __global__ __launch_bounds__(kIlvThreads) void lanes_interleave_kernel(const uin
         total += words[t];
         maxw = max(maxw, words[t]);
     }
-    for (uint32_t r0 = 0; r0 < maxw; r0 += kRoundTile) {
-        const uint32_t rn = min(kRoundTile, maxw - r0);
-        for (uint32_t i = tid; i < rn; i += kIlvThreads) {
-            const uint32_t r = r0 + i;
+    for (uint32_t r0 = blockIdx.y * kRoundTile; r0 < maxw; r0 += gridDim.y * kRoundTile) {
+        uint32_t v[kSlots][2];
+#pragma unroll
+        for (uint32_t k = 0; k < kSlots; ++k) {
+            const uint32_t t = t0 + k;
+            // slot t holds lane_map[t]'s stream (identity without a map)
+            const uint32_t* src = reinterpret_cast<const uint32_t*>(
+                work + (c * 32 + (lane_map ? lane_map[c * 32 + t] : t)) * lane_slot);
+#pragma unroll
+            for (uint32_t h = 0; h < 2; ++h) {
+                const uint32_t r = r0 + kWave * h + l;
+                v[k][h] = r < words[t] ? src[r] : 0u;
+            }
+        }
+        if (tid <= kRoundTile) {
+            const uint32_t r = r0 + tid;
             uint32_t base = 0, mask = 0;
             for (uint32_t u = 0; u < 32; ++u) {
                 const uint32_t wu = words[u];
                 base += wu < r ? wu : r;
                 mask |= (wu > r ? 1u : 0u) << u;
             }
-            rbase[i] = base;
-            rmask[i] = mask;
+            rbase[tid] = base;
+            if (tid < kRoundTile) rmask[tid] = mask;
         }
         __syncthreads();
-        for (uint32_t j = tid; j < 32 * rn; j += kIlvThreads) {
-            const uint32_t t = j / rn, i = j - t * rn, r = r0 + i;
-            if (r >= words[t]) continue;
-            const uint32_t pos = rbase[i] + __builtin_popcount(rmask[i] & ((1u << t) - 1u));
-            // slot t holds lane_map[t]'s stream (identity without a map)
-            const uint8_t* src = work + (c * 32 + (lane_map ? lane_map[c * 32 + t] : t)) * lane_slot;
-            const uint64_t len = col_len[c * 32 + t];
-            uint32_t v = *reinterpret_cast<const uint32_t*>(src + 4ull * r);
-            const uint64_t have = len - 4ull * r;       // bytes of this word inside the stream
-            if (have < 4) v &= (1u << (8 * have)) - 1u;
-            dst[pos] = v;
+        const uint32_t first = rbase[0], count = rbase[kRoundTile] - first;
+#pragma unroll
+        for (uint32_t k = 0; k < kSlots; ++k) {
+            const uint32_t t = t0 + k;
+#pragma unroll
+            for (uint32_t h = 0; h < 2; ++h) {
+                const uint32_t i = kWave * h + l, r = r0 + i;
+                if (r < words[t]) {
+                    const uint32_t have = bytes[t] - 4 * r;       // bytes of this word inside the stream
+                    const uint32_t p = rbase[i] - first + __builtin_popcount(rmask[i] & ((1u << t) - 1u));
+                    tile[p + p / 32] = have < 4 ? v[k][h] & ((1u << (8 * have)) - 1u) : v[k][h];
+                }
+            }
         }
+        __syncthreads();
+        for (uint32_t p = tid; p < count; p += kIlvThreads) dst[first + p] = tile[p + p / 32];
         __syncthreads();
     }
-    const uint64_t clen = chunk_len[c];
-    for (uint64_t q = total + tid; q < clen / 4; q += kIlvThreads) dst[q] = 0;
+    if (blockIdx.y == 0) {
+        const uint64_t clen = chunk_len[c];
+        for (uint64_t q = total + tid; q < clen / 4; q += kIlvThreads) dst[q] = 0;
+    }
+}
+
+inline dim3 interleave_grid(uint64_t n, uint64_t lane_slot) {
+    const uint64_t tiles = (lane_slot / 4 + kRoundTile - 1) / kRoundTile, parts = (kIlvGroups + n - 1) / n;
+    return dim3((uint32_t)n, (uint32_t)(parts < tiles ? parts : tiles));
 }
 
 }  // namespace

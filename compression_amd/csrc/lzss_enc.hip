@@ -286,7 +286,7 @@ int lzss_compress(const void* in, uint64_t in_bytes, uint64_t chunk, void* work,
     if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lzss_rank_kernel launch");
     hipLaunchKernelGGL(lanes_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, chunk_len, n, blk_off, nullptr, ~0ull);
     if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lanes_scan_kernel launch");
-    hipLaunchKernelGGL(lanes_interleave_kernel, dim3((uint32_t)n), dim3(kIlvThreads), 0, s,
+    hipLaunchKernelGGL(lanes_interleave_kernel, interleave_grid(n, slot), dim3(kIlvThreads), 0, s,
                        static_cast<const uint8_t*>(w), slot, col_len, blk_off, chunk_len, col_map,
                        static_cast<uint8_t*>(payload));
     return record_hip(hipGetLastError(), "lanes_interleave_kernel launch");
