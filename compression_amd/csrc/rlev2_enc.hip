@@ -25,6 +25,8 @@
 // chunks: 0.42 ms, bound by the groups' dependent ballots and LDS steps at 20
 // waves a CU (24.3 ms with one lane encoding each stream).  The scan and the
 // interleave are the shared lane-encoder kernels (lanes_enc_dev.h).
+#include <type_traits>
+
 #include "lanes_enc_dev.h"
 #include "mdz_device.h"
 #include "mdz_internal.h"
@@ -129,7 +131,7 @@ struct Group {
     template <class F> MDZ_DEV bool any_pair(F f) const {
         return ((__ballot(f(p0, a0)) & m0 & ~1ull) | (__ballot(f(p1, a1)) & m1)) != 0;
     }
-    // The width code that `below` of the n codes (c0, c1 per lane) lie above.
+    // The largest width code that more than `below` of the n codes (c0, c1 per lane) reach.
     MDZ_DEV uint32_t code_at(uint32_t c0, uint32_t c1, uint32_t below) const {
         uint32_t c = 0;
 #pragma unroll
@@ -140,8 +142,16 @@ struct Group {
         }
         return c;
     }
+    // How many of the codes are at least c.
+    MDZ_DEV uint32_t at_least(uint32_t c0, uint32_t c1, uint32_t c) const {
+        return (uint32_t)__popcll(__ballot(c0 >= c) & m0) + (uint32_t)__popcll(__ballot(c1 >= c) & m1);
+    }
+    MDZ_DEV uint32_t most(uint32_t c0, uint32_t c1) const {
+        const uint32_t l = lane_id();
+        return wave_max_u32(max(l < n ? c0 : 0u, 64 + l < n ? c1 : 0u));
+    }
     // Values above the p-th percentile, as the reference counts them.
-    MDZ_DEV uint32_t above(uint32_t p) const { return p == 100 ? 0 : (n * (100 - p) - 1) / 100 + 1; }
+    MDZ_DEV uint32_t above(uint32_t p) const { return (n * (100 - p) - 1) / 100 + 1; }
 };
 
 // The lane stream's output: `bits` bits staged (big-endian words, zero past
@@ -164,9 +174,11 @@ struct Sink {
             const uint64_t hi = top >> sh;
             const uint32_t lo = sh ? (uint32_t)top << (32 - sh) : 0u;
             uint32_t* s = stage + (at >> 5);
-            if ((uint32_t)(hi >> 32)) atomicOr(s, (uint32_t)(hi >> 32));
-            if ((uint32_t)hi) atomicOr(s + 1, (uint32_t)hi);
-            if (lo) atomicOr(s + 2, lo);
+            atomicOr(s, (uint32_t)(hi >> 32));
+            if (w + sh > 32) {
+                atomicOr(s + 1, (uint32_t)hi);
+                if (w + sh > 64) atomicOr(s + 2, lo);
+            }
         }
     }
     // A field of the whole wave's: v, bytes long.
@@ -299,16 +311,19 @@ MDZ_DEV void literals(Sink& o, const Group& g) {
             return;
         }
     }
-    const uint32_t code100 = g.code_at(c0, c1, 0);
+    const uint32_t code100 = g.most(c0, c1);
     if (g.n > kMinRepeat && !narrow) {
-        const uint32_t b100 = code_width(code100), b90 = code_width(g.code_at(c0, c1, g.above(90)));
-        if (b100 - b90 > 1) {
+        // the 90th percentile's width is over 1 below the largest: too few
+        // values reach the widths that are not (widths step by 1 up to 24,
+        // code 23, and by 2 or more beyond)
+        const uint32_t near = code100 < 24 ? max(code100, 1u) - 1 : code100;
+        if (g.at_least(c0, c1, near) <= g.above(90)) {
             const uint32_t l = lane_id();
             const uint64_t base = wave_min_u64(min(l < g.n ? g.a0 : ~0ull, 64 + l < g.n ? g.a1 : ~0ull));
             const uint32_t d0 = width_code(bit_length(g.a0 - base)), d1 = width_code(bit_length(g.a1 - base));
-            const uint32_t r95 = code_width(g.code_at(d0, d1, g.above(95))), r100 = code_width(g.code_at(d0, d1, 0));
-            if (r100 != r95) {
-                patched(o, g, base, r95, r100);
+            const uint32_t r100 = g.most(d0, d1);
+            if (g.at_least(d0, d1, r100) <= g.above(95)) {
+                patched(o, g, base, code_width(g.code_at(d0, d1, g.above(95))), code_width(r100));
                 return;
             }
         }
@@ -332,15 +347,46 @@ MDZ_DEV uint64_t chunk_value(const uint8_t* in, uint64_t in_bytes, uint64_t base
     return v;
 }
 
-template <class LT>
+// Values [s, end) of lane t of the chunk at byte `base` to val[0, end - s).
+// Where every value is whole, aligned and its line a power of two, eight loads
+// a lane are in flight.
+template <int EB, class LT>
+MDZ_DEV void load_values(LT* val, const uint8_t* in, uint64_t in_bytes, uint64_t base, uint64_t chunk, uint32_t ru,
+                         uint32_t t, uint32_t s, uint32_t end) {
+    typedef typename std::conditional<EB == 8, uint64_t, typename std::conditional<EB == 4, uint32_t,
+            typename std::conditional<EB == 2, uint16_t, uint8_t>::type>::type>::type E;
+    const uint32_t l = lane_id();
+    if (base + chunk <= in_bytes && ((uintptr_t)(in + base) & (EB - 1)) == 0 && (ru & (ru - 1)) == 0) {
+        const E* v = reinterpret_cast<const E*>(in + base);
+        const uint32_t sh = 31 - __builtin_clz(ru);
+        for (uint32_t q0 = s; q0 < end; q0 += 8 * kWave) {
+            E x[8];
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i) {
+                const uint32_t q = min(q0 + i * kWave + l, end - 1);
+                x[i] = v[((uint64_t)(q >> sh) * 32 + t) << sh | (q & (ru - 1))];
+            }
+#pragma unroll
+            for (uint32_t i = 0; i < 8; ++i)
+                if (q0 + i * kWave + l < end) val[q0 + i * kWave + l - s] = (LT)x[i];
+        }
+        return;
+    }
+    for (uint32_t q = s + l; q < end; q += kWave) {
+        const uint32_t line = q / ru;
+        val[q - s] = (LT)chunk_value(in, in_bytes, base, ((uint64_t)line * 32 + t) * ru + (q - line * ru), EB);
+    }
+}
+
+template <int EB>
 __global__ __launch_bounds__(kWave) void rlev2_encode_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes,
-                                                             uint64_t n_chunks, uint64_t chunk, uint32_t eb,
-                                                             uint32_t ru, uint64_t lane_slot,
-                                                             uint8_t* __restrict__ work,
+                                                             uint64_t n_chunks, uint64_t chunk, uint32_t ru,
+                                                             uint64_t lane_slot, uint8_t* __restrict__ work,
                                                              uint64_t* __restrict__ col_len) {
+    typedef typename std::conditional<EB == 8, uint64_t, uint32_t>::type LT;
     __shared__ V2EncLds<LT> S;
     constexpr uint32_t kVals = V2EncLds<LT>::kVals;
-    const uint32_t l = lane_id(), nv = (uint32_t)(chunk / eb / 32);
+    const uint32_t l = lane_id(), nv = (uint32_t)(chunk / EB / 32);
     for (uint64_t unit = blockIdx.x; unit < lane_units(n_chunks); unit += gridDim.x) {
         uint64_t c;
         uint32_t t;
@@ -353,10 +399,7 @@ __global__ __launch_bounds__(kWave) void rlev2_encode_kernel(const uint8_t* __re
                 wave_sync();
                 w0 = s;
                 end = min(nv - s, kVals) + s;
-                for (uint32_t q = s + l; q < end; q += kWave) {
-                    const uint32_t line = q / ru;
-                    S.val[q - s] = (LT)chunk_value(in, in_bytes, c * chunk, ((uint64_t)line * 32 + t) * ru + (q - line * ru), eb);
-                }
+                load_values<EB>(S.val, in, in_bytes, c * chunk, chunk, ru, t, s, end);
                 wave_sync();
             }
             const uint32_t have = min(nv - s, kMaxLit), at = s - w0 + l;
@@ -422,12 +465,10 @@ int rlev2_compress(const void* in, uint64_t in_bytes, uint64_t chunk, uint32_t e
     const uint64_t slot = v2_lane_slot(chunk, eb);
     uint64_t* chunk_len = reinterpret_cast<uint64_t*>(static_cast<uint8_t*>(work) + n * 32 * slot);
     const dim3 grid = lane_grid(n), block(kWave);
-    if (eb <= 4)
-        hipLaunchKernelGGL(rlev2_encode_kernel<uint32_t>, grid, block, 0, s, static_cast<const uint8_t*>(in), in_bytes,
-                           n, chunk, eb, ru, slot, static_cast<uint8_t*>(work), col_len);
-    else
-        hipLaunchKernelGGL(rlev2_encode_kernel<uint64_t>, grid, block, 0, s, static_cast<const uint8_t*>(in), in_bytes,
-                           n, chunk, eb, ru, slot, static_cast<uint8_t*>(work), col_len);
+    auto encode = eb == 1 ? rlev2_encode_kernel<1> : eb == 2 ? rlev2_encode_kernel<2>
+                : eb == 4 ? rlev2_encode_kernel<4> : rlev2_encode_kernel<8>;
+    hipLaunchKernelGGL(encode, grid, block, 0, s, static_cast<const uint8_t*>(in), in_bytes, n, chunk, ru, slot,
+                       static_cast<uint8_t*>(work), col_len);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return record_hip(e, "rlev2_encode_kernel launch");
     hipLaunchKernelGGL(lanes_size_kernel, dim3((uint32_t)((n + kSizeChunks - 1) / kSizeChunks)), dim3(kSizeThreads), 0, s,
