@@ -13,17 +13,18 @@
 //
 // One wave encodes one lane stream.  The stream's bytes and an index of its
 // positions live in LDS: `slot` lists the positions bucket by bucket (9 hash
-// bits of 3 bytes), ascending inside a bucket.  At each token the 64 lanes
-// compare 64 candidates of the token's bucket at once, oldest first; a search
-// ends when no younger candidate can be longer.  Only the positions the greedy
-// parse reaches are searched, and what the whole wave shares (position, best
-// match, output offset) is scalar.  What bounds it is the dependent chain of
-// LDS reads and scalar steps from one token to the next, so what counts is how
-// many streams a CU holds: 7.4 KiB of LDS each up to 2048 lane bytes (64 KiB
-// chunks), 14 KiB beyond.  Lanes over 4096 bytes are indexed in windows of
-// 4096 positions that advance by 2048.  64 MiB in 64 KiB chunks: 3.4 ms, VALU
-// issue 66 % busy (412 ms with one lane per stream and chains in global
-// memory; 6.5 ms with half a wave per stream and misaligned LDS reads).
+// bits of 3 bytes), ascending inside a bucket.  A step searches two
+// neighbouring positions, each half of the wave comparing 32 candidates of
+// its position's bucket at once, oldest first; if the first becomes a literal
+// the second's token follows in the same step, which about half of all tokens
+// do.  A search ends when no younger candidate can be longer.  Only positions
+// that the greedy parse reaches, and their successors, are searched, and what
+// the whole wave shares (position, best matches, output offset) is scalar.
+// What bounds it is instruction issue at the waves that LDS allows: 7.4 KiB
+// per stream up to 2048 lane bytes (64 KiB chunks), 14 KiB beyond.  Lanes over
+// 4096 bytes are indexed in windows of 4096 positions that advance by 2048.
+// 64 MiB in 64 KiB chunks: 2.7 ms (3.4 ms with one position a step; 412 ms with
+// one lane per stream and chains in global memory).
 //
 // A second kernel ranks a chunk's 32 lanes by length (descending, ties to
 // the higher lane id) into col_map; the shared kernels scan the chunk
@@ -38,13 +39,15 @@ namespace {
 constexpr uint32_t kHist = 2048, kMinLen = 3, kMaxLen = 34, kLenBits = 5;
 constexpr uint32_t kHashBits = 9, kBuckets = 1u << kHashBits;
 
+constexpr uint32_t kHalf = 32;                  // lanes that search one position
+
 // One lane stream's window: kCap positions and the bytes a match at the last
 // of them can reach.
 template <uint32_t kCap>
 struct LzStream {
     static constexpr bool kOld = kCap > kHist;  // candidates can be out of reach
     uint32_t data[(kCap + 64) / 4];
-    uint16_t slot[kCap + kWave];                // positions by bucket, ascending (the tail is read, not used)
+    uint16_t slot[kCap + kWave];                // positions by bucket, ascending; then kWave that are no candidates
     uint32_t bound[kBuckets / 2 + 1];           // u16: bucket h's slots are [bound[h], bound[h + 1])
     uint16_t first[kOld ? kBuckets : 2];        // first slot still within reach
 };
@@ -60,8 +63,11 @@ MDZ_DEV uint64_t lds_u64(const uint32_t* w, uint32_t p) {
     const uint32_t k = p >> 2, w0 = w[k], w1 = w[k + 1], w2 = w[k + 2];
     return (uint64_t)alignbyte(w2, w1, p & 3) << 32 | alignbyte(w1, w0, p & 3);
 }
-MDZ_DEV uint32_t lz_hash(uint32_t v) { return ((v & 0xFFFFFFu) * 2654435761u) >> (32 - kHashBits); }
-MDZ_DEV uint32_t uniform(uint32_t v) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)v); }
+// Of the low 3 bytes (a 24-bit multiply takes no others).
+MDZ_DEV uint32_t lz_hash(uint32_t v) { return (uint32_t)__umul24(v, 0x9E3779u) >> (32 - kHashBits); }
+// Zero bits below the lowest set one; all ones if there is none (v_ffbl_b32).
+MDZ_DEV uint32_t ctz_or_max(uint32_t v) { return v ? (uint32_t)__builtin_ctz(v) : 0xFFFFFFFFu; }
+MDZ_DEV uint32_t add_sat(uint32_t a, uint32_t b) { return __builtin_elementwise_add_sat(a, b); }
 MDZ_DEV uint32_t lane_value_at(uint32_t v, uint32_t lane) {
     return (uint32_t)__builtin_amdgcn_readlane((int)v, (int)lane);
 }
@@ -106,9 +112,11 @@ MDZ_DEV void lz_index(LzStream<kCap>& S, uint32_t p0, uint32_t p1, uint32_t l) {
     // each slot given out moves its bucket's first slot: to the bucket's end
     for (uint32_t p = p0 + l; p < p1; p += kWave) S.slot[bump(lz_hash(lds_u32(S.data, p)))] = (uint16_t)p;
     wave_sync();
+    // steps past the list's end read positions that are no candidates
+    const uint32_t ns = p1 > p0 ? p1 - p0 : 0;
+    S.slot[ns + l] = (uint16_t)(kCap - 1);
     // The 64 positions of one step may take their bucket's slots in any
     // order: put neighbours in order until none is out of it.
-    const uint32_t ns = p1 > p0 ? p1 - p0 : 0;
     for (;;) {
         bool moved = false;
 #pragma unroll
@@ -133,7 +141,7 @@ __global__ __launch_bounds__(kWave) void lzss_encode_kernel(const uint8_t* __res
                                                             uint8_t* __restrict__ work,
                                                             uint32_t* __restrict__ lane_len) {
     __shared__ LzStream<kCap> S;
-    const uint32_t l = lane_id();
+    const uint32_t l = lane_id(), half = l / kHalf;
     const uint16_t* bounds = reinterpret_cast<const uint16_t*>(S.bound);
     const uint32_t n = (uint32_t)(chunk / 32);
     for (uint64_t unit = blockIdx.x; unit < lane_units(n_chunks); unit += gridDim.x) {
@@ -153,58 +161,88 @@ __global__ __launch_bounds__(kWave) void lzss_encode_kernel(const uint8_t* __res
             // position 0 is never a candidate, nor one with under 3 bytes left
             lz_index<kCap>(S, w0 ? 0u : 1u, min(stop, left >= kMinLen ? left - (kMinLen - 1) : 0u), l);
             while (cur < stop) {
-                const uint64_t here = lds_u64(S.data, cur);
-                const uint32_t look = min(left - cur, kMaxLen);      // longest match left
-                uint32_t len = 0, from = 0;
-                uint32_t h = lz_hash((uint32_t)here);
-                uint32_t i = uniform(bounds[h]);
-                const uint32_t e = look >= kMinLen ? uniform(bounds[h + 1]) : 0u;
-                if constexpr (LzStream<kCap>::kOld) i = uniform(S.first[h]);
-                for (; i < e; i += kWave) {
-                    const uint32_t q = S.slot[i + l];
-                    const uint32_t qa = q & (kCap - 1);                // slots past the list hold anything
-                    const uint64_t x = lds_u64(S.data, qa) ^ here;
-                    const uint32_t cap = min(cur - q, look);
-                    const bool ok = i + l < e && cur - 1 - q < kHist - 1;   // older, and within reach
-                    uint32_t f = x ? (uint32_t)__builtin_ctzll(x) >> 3 : 8u;
-                    if (__ballot(ok && !x && cap > 8 && cap > len)) {
-                        bool run = ok && !x && cap > 8;
+                const uint32_t p = cur + half;
+                const uint64_t here = lds_u64(S.data, p);
+                const int32_t look = min((int32_t)(left - p), (int32_t)kMaxLen);  // longest match left
+                const uint32_t h = lz_hash((uint32_t)here);
+                uint32_t i = bounds[h];
+                if constexpr (LzStream<kCap>::kOld) i = S.first[h];
+                i += l % kHalf;
+                const uint32_t e = bounds[h + 1];
+                uint32_t len[2] = {0, 0}, from[2] = {0, 0};
+                uint32_t least = kMinLen - 1;                // a match has to be longer
+                for (;;) {
+                    // Slots past the bucket's list hold positions of other 3 bytes,
+                    // or none older than p: neither passes.
+                    const uint32_t q = S.slot[i];
+                    const int32_t cap = min((int32_t)(p - q), look);
+                    const uint64_t x = lds_u64(S.data, q) ^ here;
+                    // equal bytes, then at most cap; beyond 8 only if all 8 are equal
+                    const uint32_t lo = ctz_or_max((uint32_t)x), hi = ctz_or_max((uint32_t)(x >> 32));
+                    int32_t f = min((int32_t)(min(lo, add_sat(hi, 32u)) >> 3), cap);
+                    if constexpr (LzStream<kCap>::kOld) f = p - q < kHist ? f : 0;
+                    bool run = f > 8;
+                    if (__ballot(run)) {
                         for (uint32_t j = 8; j < kMaxLen; j += 8) {
-                            const uint64_t y = lds_u64(S.data, qa + j) ^ lds_u64(S.data, cur + j);
-                            f = !run ? f : y ? j + ((uint32_t)__builtin_ctzll(y) >> 3) : j + 8;
-                            run = run && !y && cap > j + 8;
+                            const uint64_t y = lds_u64(S.data, q + j) ^ lds_u64(S.data, p + j);
+                            const int32_t g = (int32_t)(j + (y ? (uint32_t)__builtin_ctzll(y) >> 3 : 8u));
+                            f = run ? min(g, cap) : f;
+                            run = run && !y && cap > (int32_t)(j + 8);
                             if (!__ballot(run)) break;
                         }
                     }
-                    f = ok ? min(f, cap) : 0u;
-                    // the oldest of the longest: each better one in turn
-                    for (uint64_t m = __ballot(f > max(len, kMinLen - 1)); m; m = __ballot(f > len)) {
-                        const uint32_t lane = (uint32_t)__builtin_ctzll(m);
-                        len = lane_value_at(f, lane);
-                        from = lane_value_at(q, lane);
+                    // the oldest of the longest, in each half: each better one in turn
+                    uint64_t m = __ballot(f > (int32_t)least);
+#pragma unroll
+                    for (uint32_t k = 0; k < 2; ++k) {
+                        uint32_t mk = (uint32_t)(k ? m >> 32 : m);
+                        while (mk) {
+                            const uint32_t lane = kHalf * k + (uint32_t)__builtin_ctz(mk);
+                            len[k] = lane_value_at((uint32_t)f, lane);
+                            from[k] = lane_value_at(q, lane);
+                            const uint64_t better = __ballot(f > (int32_t)len[k]);
+                            mk = (uint32_t)(k ? better >> 32 : better);
+                        }
                     }
+                    // the next 32: if the last of these is in the list's middle and older
+                    const uint64_t more = __ballot(i + 1 < e && q < p);
+                    bool go0 = (more >> (kHalf - 1)) & 1, go1 = more >> (kWave - 1);
                     if constexpr (LzStream<kCap>::kOld) {
                         // a step wholly out of reach stays so for later positions
-                        if (i + kWave <= e && __ballot(q + kHist <= cur) == ~0ull && l == 0) S.first[h] = (uint16_t)(i + kWave);
+                        const uint64_t old = __ballot(q + kHist <= p);
+                        if (go0 && (uint32_t)old == ~0u && l == kHalf - 1) S.first[h] = (uint16_t)(i + 1);
+                        if (go1 && (uint32_t)(old >> 32) == ~0u && l == kWave - 1) S.first[h] = (uint16_t)(i + 1);
                     }
-                    if (len >= look || !(__ballot(q < cur) >> (kWave - 1))) break;
+                    const uint32_t most = min(left - cur, kMaxLen);
+                    go0 = go0 && len[0] < most;
+                    go1 = go1 && len[1] < min(left - cur - 1, kMaxLen) && (go0 || !len[0]);
+                    if (!go0 && !go1) break;
+                    // a half that is done stays where it is and takes no more
+                    const bool go = half ? go1 : go0;
+                    least = go ? max(half ? len[1] : len[0], kMinLen - 1) : kWave;
+                    i += go ? kHalf : 0;
                 }
-                if (len == 0) {
-                    if (l == 0) out[o] = (uint8_t)here;
-                    flags |= 1u << ntok;
-                    o += 1;
-                    cur += 1;
-                } else {
-                    const uint16_t v = (uint16_t)((cur - from) << kLenBits | (len - kMinLen));
-                    if (l == 0) __builtin_memcpy(out + o, &v, 2);
-                    o += 2;
-                    cur += len;
-                }
-                if (++ntok == 8) {              // the next group's flag byte is reserved at once
-                    if (l == 0) out[flag_at] = (uint8_t)flags;
-                    flags = 0;
-                    ntok = 0;
-                    flag_at = o++;
+                // one token, and the successor's if it is a literal
+#pragma unroll
+                for (uint32_t k = 0; k < 2; ++k) {
+                    if (len[k] == 0) {
+                        if (l == kHalf * k) out[o] = (uint8_t)here;
+                        flags |= 1u << ntok;
+                        o += 1;
+                        cur += 1;
+                    } else {
+                        const uint16_t v = (uint16_t)((cur - from[k]) << kLenBits | (len[k] - kMinLen));
+                        if (l == 0) __builtin_memcpy(out + o, &v, 2);
+                        o += 2;
+                        cur += len[k];
+                    }
+                    if (++ntok == 8) {          // the next group's flag byte is reserved at once
+                        if (l == 0) out[flag_at] = (uint8_t)flags;
+                        flags = 0;
+                        ntok = 0;
+                        flag_at = o++;
+                    }
+                    if (k == 0 && (len[0] || cur >= stop)) break;
                 }
                 if constexpr (LzStream<kCap>::kOld) wave_sync();        // first[] before its next reader
             }
@@ -220,7 +258,7 @@ __global__ __launch_bounds__(kWave) void lzss_encode_kernel(const uint8_t* __res
 
 // Sorted slot of lane t: longer lanes first, equal lengths by higher lane id.
 // Half a wave per chunk.
-constexpr uint32_t kHalf = 32, kRankThreads = 256, kRankChunks = kRankThreads / kHalf;
+constexpr uint32_t kRankThreads = 256, kRankChunks = kRankThreads / kHalf;
 
 __global__ __launch_bounds__(kRankThreads) void lzss_rank_kernel(const uint32_t* __restrict__ lane_len, uint64_t n_chunks,
                                                                  uint64_t* __restrict__ col_len,
