@@ -24,6 +24,8 @@
 //      blk_off.
 //   3. The lane streams are interleaved in the round-robin order of
 //      encoder.h:564-588 (lanes_enc_dev.h).
+#include <type_traits>
+
 #include "lanes_enc_dev.h"
 #include "mdz_device.h"
 #include "mdz_internal.h"
@@ -116,6 +118,8 @@ __global__ __launch_bounds__(kWave) void rlev1_encode_kernel(const uint8_t* __re
                                                              uint64_t lane_slot, uint8_t* __restrict__ work,
                                                              uint64_t* __restrict__ col_len) {
     typedef typename Wide<EB>::T T;
+    typedef typename std::conditional<EB == 8, uint64_t, typename std::conditional<EB == 4, uint32_t,
+            typename std::conditional<EB == 2, uint16_t, uint8_t>::type>::type>::type Elem;
     __shared__ uint32_t stage[kStageBytes / 4 + 1];
     const uint32_t l = lane_id(), n = (uint32_t)(chunk / 32 / EB);
     const bool pow2 = (line & (line - 1)) == 0;
@@ -124,9 +128,17 @@ __global__ __launch_bounds__(kWave) void rlev1_encode_kernel(const uint8_t* __re
         uint64_t c;
         uint32_t t;
         if (!lane_of_unit(unit, n_chunks, c, t)) continue;
-        auto value = [&](uint32_t k) -> T {               // lane value k: byte k*EB sits in line t + 32*(k*EB / line)
+        // lane value k: byte k*EB sits in line t + 32*(k*EB / line).  A chunk
+        // inside the input, aligned, with lines of a power of two: one load.
+        const uint8_t* src = in + c * chunk;
+        const bool plain = pow2 && (c + 1) * chunk <= in_bytes && ((uintptr_t)src & (EB - 1)) == 0;
+        auto value = [&](uint32_t k) -> T {
+            if (plain) {
+                const uint32_t o = min(k, n - 1) * EB;
+                return *reinterpret_cast<const Elem*>(src + ((((uint64_t)(o >> shift) * 32 + t) << shift) | (o & (line - 1))));
+            }
             if (k >= n) return 0;
-            const uint32_t o = k * EB, r = pow2 ? o >> shift : o / line, j = o - r * line;
+            const uint32_t o = k * EB, r = o / line, j = o - r * line;
             return (T)load_elem(in, in_bytes, c * chunk + (t + 32ull * r) * line + j, EB);
         };
         LaneStage w{reinterpret_cast<uint8_t*>(stage), work + (c * 32 + t) * lane_slot, 0, 0};
