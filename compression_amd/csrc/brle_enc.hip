@@ -17,17 +17,20 @@
 // So any stretch of segments maps n to n' by {shift; the result for a shifted
 // n below 126, for 126, for 127}, 29 bits, and such maps compose: the state
 // machine is a prefix scan.  Per window of 32 KiB (32 bytes a thread):
-//   1. each thread marks where segments start in its bytes; a scan finds the
-//      segment open before them.  A segment belongs to the thread that sees
-//      the next one start, so no thread looks ahead;
-//   2. it composes its segments' maps, and a scan gives the literals pending
-//      before its first segment;
+//   1. each thread marks where segments start in its bytes, and a scan packs
+//      those positions into a list: each ends the segment before it, so no
+//      thread looks ahead.  The list's segments are dealt out evenly, the same
+//      number to every thread, whatever bytes they cover;
+//   2. each thread composes its segments' maps, and a scan gives the literals
+//      pending before its first segment;
 //   3. it counts the bytes its segments add, and a scan places them;
 //   4. it writes them to the LDS copy of the output, which the workgroup
 //      stores 16 bytes at a time.  A group's header byte is reserved with its
 //      first literal and written by the segment that ends the group.
-// The scans' latency bounds it (three barriers a window and about 1000 vector
-// instructions a wave), so a workgroup is as wide as the hardware allows.
+// Vector issue and the scans' latency bound it (four barriers a window), so a
+// workgroup is as wide as the hardware allows.  64 MiB of mean run length 12
+// in 256 KiB chunks: 96 us for this kernel (161 us with each thread taking the
+// segments that end in its own bytes, 22.0 ms with one lane walking a chunk).
 // Groups go to a per-chunk slot of the work buffer; a scan kernel turns the
 // chunk sizes into ptr[] and a shift kernel packs the slots into `data`.
 #include "mdz_device.h"
@@ -45,6 +48,7 @@ constexpr uint32_t kStage = kWin + kWin / 32;   // staged output bytes of a wind
 struct EncLds {
     alignas(16) uint32_t in[kWin / 4];
     alignas(16) uint32_t out[kStage / 4 + 8];
+    uint16_t list[kWin];                        // window offsets where a segment ends
     uint32_t part[3][kEncWaves];
 };
 
@@ -85,15 +89,6 @@ MDZ_DEV uint32_t wave_incl_maps(uint32_t v) {
     v = map_then(dpp_src<0x118, 0xf, 0u>(v), v);
     v = map_then(dpp_src<0x142, 0xa, 0u>(v), v);
     v = map_then(dpp_src<0x143, 0xc, 0u>(v), v);
-    return v;
-}
-MDZ_DEV uint32_t wave_incl_max_u32(uint32_t v) {
-    v = max(v, dpp_src<0x111, 0xf, 0u>(v));
-    v = max(v, dpp_src<0x112, 0xf, 0u>(v));
-    v = max(v, dpp_src<0x114, 0xf, 0u>(v));
-    v = max(v, dpp_src<0x118, 0xf, 0u>(v));
-    v = max(v, dpp_src<0x142, 0xa, 0u>(v));
-    v = max(v, dpp_src<0x143, 0xc, 0u>(v));
     return v;
 }
 // The value of the lane below; `first` in lane 0.
@@ -156,18 +151,21 @@ MDZ_DEV int32_t write_segment(Put put, int32_t o, uint32_t& n, uint32_t L, uint3
 
 // Exclusive scan over the workgroup through part[16]: `incl` is the wave's
 // inclusive scan, `carry` comes before the workgroup's first thread and takes
-// in its last.  One barrier.
+// in its last.  One barrier; every row of 16 lanes then scans the parts.
 template <class Then>
 MDZ_DEV uint32_t block_scan(uint32_t* part, uint32_t incl, uint32_t& carry, Then then) {
+    static_assert(kEncWaves == 16, "the parts fill a row");
     const uint32_t wave = threadIdx.x / kWave;
     if (lane_id() == kWave - 1) part[wave] = incl;
     __syncthreads();
-    uint32_t before = carry, all = carry;
-    for (uint32_t w = 0; w < kEncWaves; ++w) {
-        all = then(all, part[w]);
-        if (w + 1 == wave) before = all;
-    }
-    carry = all;
+    uint32_t v = part[lane_id() & 15];
+    v = then(dpp_src<0x111, 0xf, 0u>(v), v);              // 0 is every map's identity
+    v = then(dpp_src<0x112, 0xf, 0u>(v), v);
+    v = then(dpp_src<0x114, 0xf, 0u>(v), v);
+    v = then(dpp_src<0x118, 0xf, 0u>(v), v);
+    const uint32_t below = (uint32_t)__builtin_amdgcn_readlane((int)v, wave ? (int)wave - 1 : 0);
+    const uint32_t before = wave ? then(carry, below) : carry;
+    carry = then(carry, (uint32_t)__builtin_amdgcn_readlane((int)v, 15));
     return then(before, from_below(incl, 0));
 }
 
@@ -185,6 +183,7 @@ __global__ __launch_bounds__(kEncThreads) void brle_encode_kernel(const uint8_t*
     const uint8_t* in8 = reinterpret_cast<const uint8_t*>(S.in);
     uint8_t* out8 = reinterpret_cast<uint8_t*>(S.out);
     const uint32_t skew = (uint32_t)((uintptr_t)src & 3);
+    auto plus = [](uint32_t a, uint32_t b) { return a + b; };
     uint32_t open = 0;                          // start of the segment open before the window
     uint32_t state = 0;                         // map of the segments before the window: pending literals
     uint32_t last = 0x100;                      // the byte before the window
@@ -231,16 +230,21 @@ __global__ __launch_bounds__(kEncThreads) void brle_encode_kernel(const uint8_t*
         }
         if (w0 + t == 0) mask |= 1;             // the chunk's first byte opens a segment
         mask = at >= wl ? 0 : wl - at >= kPer ? mask : mask & ((1u << (wl - at)) - 1);
-        const uint32_t newest = mask ? w0 + at + 31 - __builtin_clz(mask) : 0;
-        const uint32_t prev0 = block_scan(S.part[0], wave_incl_max_u32(newest), open,
-                                          [](uint32_t a, uint32_t b) { return max(a, b); });
         // the segments that end in these bytes (position 0 ends none)
         const uint32_t ends = w0 + t == 0 ? mask & ~1u : mask;
+        uint32_t count = 0;
+        {
+            const uint32_t mine = (uint32_t)__builtin_popcount(ends);
+            uint32_t i = block_scan(S.part[0], wave_incl_scan_u32(mine), count, plus);
+            for (uint32_t m = ends; m; m &= m - 1) S.list[i++] = (uint16_t)(at + (uint32_t)__builtin_ctz(m));
+        }
+        __syncthreads();
+        const uint32_t share = (count + kEncThreads - 1) / kEncThreads, s0 = min(count, t * share), s1 = min(count, s0 + share);
         auto each = [&](auto fn) {
-            uint32_t prev = prev0;
-            for (uint32_t m = ends; m; m &= m - 1) {
-                const uint32_t b = (uint32_t)__builtin_ctz(m), p = w0 + at + b;
-                fn(p - prev, at + b);
+            uint32_t prev = s0 ? w0 + S.list[s0 - 1] : open;
+            for (uint32_t i = s0; i < s1; ++i) {
+                const uint32_t o = S.list[i], p = w0 + o;
+                fn(p - prev, o);
                 prev = p;
             }
         };
@@ -252,8 +256,7 @@ __global__ __launch_bounds__(kEncThreads) void brle_encode_kernel(const uint8_t*
         uint32_t bytes = 0, n3 = n;
         each([&](uint32_t L, uint32_t) { bytes += count_segment(n3, L); });
         uint32_t total = 0;
-        const uint32_t off = block_scan(S.part[2], wave_incl_scan_u32(bytes), total,
-                                        [](uint32_t a, uint32_t b) { return a + b; });
+        const uint32_t off = block_scan(S.part[2], wave_incl_scan_u32(bytes), total, plus);
         // 4. write them.  LDS byte i holds output byte (staged & ~15) + i; what
         // does not fit there (long runs), and headers stored before, go straight out
         const uint64_t stage0 = staged & ~15ull;
@@ -270,6 +273,7 @@ __global__ __launch_bounds__(kEncThreads) void brle_encode_kernel(const uint8_t*
         int32_t o = (int32_t)off;
         each([&](uint32_t L, uint32_t p) { o = write_segment(put, o, n, L, p ? in8[p - 1] : last); });
         last = in8[wl - 1];
+        if (count) open = w0 + S.list[count - 1];
         __syncthreads();
         done += total;
         if (fits) {                             // store whole 16-byte units, keep the rest
