@@ -334,7 +334,9 @@ __global__ __launch_bounds__(kScanThreads) void brle_scan_kernel(const uint64_t*
 
 // data[ptr[c], ptr[c + 1]) = work[c * slot, ...): dword stores at aligned
 // destination addresses, each assembled from the two source dwords it spans.
-constexpr uint32_t kShiftThreads = 256;
+// Few chunks are split over `gridDim.y` workgroups each, so that the chip is
+// full (64 MiB in 256 chunks: 16 us with one workgroup per chunk).
+constexpr uint32_t kShiftThreads = 256, kShiftGroups = 2048;
 
 __global__ __launch_bounds__(kShiftThreads) void brle_shift_kernel(const uint8_t* __restrict__ work, uint64_t slot,
                                                                    const uint64_t* __restrict__ ptr,
@@ -343,19 +345,19 @@ __global__ __launch_bounds__(kShiftThreads) void brle_shift_kernel(const uint8_t
     const uint64_t d0 = ptr[c], n = ptr[c + 1] - d0;
     const uint8_t* s = work + c * slot;        // slot starts are 16-byte aligned
     uint8_t* d = data + d0;
-    const uint32_t t = threadIdx.x;
+    const uint32_t t = blockIdx.y * kShiftThreads + threadIdx.x, step = gridDim.y * kShiftThreads;
     const uint64_t head = min<uint64_t>((4 - ((uintptr_t)d & 3)) & 3, n);
-    for (uint64_t i = t; i < head; i += kShiftThreads) d[i] = s[i];
+    for (uint64_t i = t; i < head; i += step) d[i] = s[i];
     const uint64_t nw = (n - head) / 4;
     const uint32_t sk = (uint32_t)(head & 3);          // source skew of each destination dword
     const uint32_t* s4 = reinterpret_cast<const uint32_t*>(s + (head & ~3ull));
     uint32_t* d4 = reinterpret_cast<uint32_t*>(d + head);
-    for (uint64_t i = t; i < nw; i += kShiftThreads) {
+    for (uint64_t i = t; i < nw; i += step) {
         // source bytes head + 4i .. + 3 lie in dwords i and i + 1 of s4 (the
         // slot is padded, so the second read stays inside it)
         d4[i] = sk ? alignbyte(s4[i + 1], s4[i], sk) : s4[i];
     }
-    for (uint64_t i = head + 4 * nw + t; i < n; i += kShiftThreads) d[i] = s[i];
+    for (uint64_t i = head + 4 * nw + t; i < n; i += step) d[i] = s[i];
 }
 
 }  // namespace
@@ -387,7 +389,8 @@ int brle_compress(const void* in, uint64_t in_bytes, uint64_t chunk, void* work,
     if (e != hipSuccess) return record_hip(e, "brle_encode_kernel launch");
     hipLaunchKernelGGL(brle_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, sizes, n, ptr);
     if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "brle_scan_kernel launch");
-    hipLaunchKernelGGL(brle_shift_kernel, dim3((uint32_t)n), dim3(kShiftThreads), 0, s,
+    const uint64_t most = (chunk + 4 * kShiftThreads - 1) / (4 * kShiftThreads), want = (kShiftGroups + n - 1) / n;
+    hipLaunchKernelGGL(brle_shift_kernel, dim3((uint32_t)n, (uint32_t)(want < most ? want : most)), dim3(kShiftThreads), 0, s,
                        static_cast<const uint8_t*>(work), slot, ptr, static_cast<uint8_t*>(data));
     return record_hip(hipGetLastError(), "brle_shift_kernel launch");
 }
