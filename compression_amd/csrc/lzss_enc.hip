@@ -292,7 +292,9 @@ uint64_t lz_lane_slot(uint64_t chunk) {
 int lzss_compress_bound(uint64_t in_bytes, uint64_t chunk, uint64_t* n_chunks, uint64_t* work_bytes,
                         uint64_t* payload_cap) {
     // whole chunks only (a trailing partial chunk is dropped, as the reference
-    // encoder drops it); lane positions fit the u16 chains
+    // encoder drops it), at most 1 MiB.  Of the chunk * 2 bytes behind a chunk's
+    // lane slots the encoder uses 128, the lane lengths; callers' buffers keep
+    // their size.
     if (chunk == 0 || chunk % 128 || chunk > (1ull << 20) || in_bytes < chunk) return MDZ_ERR_INVALID;
     const uint64_t n = in_bytes / chunk;
     const uint64_t slot = lz_lane_slot(chunk);
