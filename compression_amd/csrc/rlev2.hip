@@ -6,8 +6,8 @@
 //
 // The decode itself is rlev2_part (rlev2_dev.h): stage, parallel header walk,
 // overlapped check and decode.  Two launch shapes:
-//   * whole chunks: one 512-thread workgroup per chunk (the LDS area sized
-//     by the largest chunk);
+//   * whole chunks: one 512-thread workgroup per chunk, or 1024 threads where
+//     only one fits a CU (the LDS area sized by the largest chunk);
 //   * lane quarters: when the caller bounds the largest quarter (8 lanes) of
 //     any chunk, one 256-thread workgroup per quarter.  The LDS area shrinks
 //     to the quarter's bytes, so several times more header walks -- the
@@ -21,11 +21,19 @@ namespace mdz {
 namespace {
 
 constexpr uint32_t kQuarterLanes = 8, kQuarterThreads = 256;
+// Where one workgroup's LDS leaves no room for a second on the CU (the caller
+// did not say how large a chunk is, or chunks are large), the workgroup is as
+// wide as the hardware allows: 16 waves stage the payload and decode the runs
+// that 8 did.  Three 128 KiB chunks of 8-byte values 42.7 -> 33.7 us, 64 MiB of
+// 4-byte values 169 -> 129 us, of bytes 469 -> 357 us.  A chunk of few values
+// has too few runs for them: 2048 of 8 bytes take 21.8 us with 512 threads and
+// 23.1 with 1024, 3072 take 25.4 and 24.1.
+constexpr uint32_t kWideThreads = 1024, kLdsPerCu = 160 * 1024, kWideValues = 3072;
 
-template <int EB>
-__global__ __launch_bounds__(kThreads) void rlev2_decode_kernel(Rlev2Args a) {
+template <int EB, uint32_t NT>
+__global__ __launch_bounds__(NT) void rlev2_decode_kernel(Rlev2Args a) {
     extern __shared__ __align__(16) uint32_t smem[];
-    rlev2_part<EB, 32, kThreads>(a, blockIdx.x, 0, smem);
+    rlev2_part<EB, 32, NT>(a, blockIdx.x, 0, smem);
 }
 
 // Block id -> (chunk, part) with the parts of a chunk on one XCD (block ids
@@ -63,9 +71,11 @@ hipError_t launch(const mdz_lanes_t& in, void* dst, uint64_t dst_bytes, int32_t*
     hipError_t e;
     if (!quarters) {
         const size_t smem = (size_t)data_cap + 16 + sizeof(Rlev2Tables<PartPool<32>::value>);
-        auto k = rlev2_decode_kernel<EB>;
+        const uint64_t bytes = dst_bytes < in.chunk_bytes ? dst_bytes : in.chunk_bytes;
+        const bool wide = 2 * smem > kLdsPerCu && bytes / EB >= kWideValues;
+        auto k = wide ? rlev2_decode_kernel<EB, kWideThreads> : rlev2_decode_kernel<EB, kThreads>;
         if ((e = set_dynamic_lds((const void*)k, smem)) != hipSuccess) return e;
-        hipLaunchKernelGGL(k, dim3((uint32_t)in.n_chunks), dim3(kThreads), smem, s, a);
+        hipLaunchKernelGGL(k, dim3((uint32_t)in.n_chunks), dim3(wide ? kWideThreads : kThreads), smem, s, a);
         return hipGetLastError();
     }
     const size_t smem = (size_t)data_cap + 16 + sizeof(Rlev2Tables<PartPool<kQuarterLanes>::value>);

@@ -139,3 +139,19 @@ def test_random_corruption_matches_oracle(gpu, seed, quarters, window):
     for ch in np.flatnonzero(ref_st == 0):
         lo, hi = ch * c.chunk, min((ch + 1) * c.chunk, c.raw_bytes)
         assert np.array_equal(got[lo:hi], ref_out[lo:hi]), ch
+
+
+# both workgroup widths: few values (under 3072 in a chunk) or room for two
+# workgroups' LDS on a CU take 512 threads, the rest 1024
+@pytest.mark.parametrize("dtype", [np.uint64, np.uint16])
+@pytest.mark.parametrize("nvals", [3071, 3072, 9000, 16384 * 3 + 5])
+@pytest.mark.parametrize("max_chunk", [0, 60_000, 66_000, 72_000, 150_000])
+def test_workgroup_widths(gpu, dtype, nvals, max_chunk):
+    eb = np.dtype(dtype).itemsize
+    x = O.gen_rlev2_i64(nvals, nvals + eb).astype(dtype)
+    c = O.rlev2_encode(x, 8192 * eb, 64, threads=4)
+    # max_chunk is a promise: the least one holds, the largest chunk being about 41 KB
+    assert np.diff(np.append(c.blk_off[:-1], np.uint64(c.payload_bytes))).max() <= 60_000
+    print(f"rlev2 decode {nvals} values of {eb} bytes, max_chunk {max_chunk}", flush=True)
+    got, st = _run(gpu, c, max_chunk=max_chunk)
+    assert (st == 0).all() and np.array_equal(got, x.view(np.uint8))
