@@ -28,7 +28,8 @@
 //      stores 16 bytes at a time.  A group's header byte is reserved with its
 //      first literal and written by the segment that ends the group.
 // Vector issue and the scans' latency bound it (four barriers a window), so a
-// workgroup is as wide as the hardware allows.  64 MiB of mean run length 12
+// workgroup is as wide as the hardware allows; chunks of at most 2 or 8 KiB get
+// one of 1 or 4 waves, with windows to match.  64 MiB of mean run length 12
 // in 256 KiB chunks: 96 us for this kernel (161 us with each thread taking the
 // segments that end in its own bytes, 22.0 ms with one lane walking a chunk).
 // Groups go to a per-chunk slot of the work buffer; a scan kernel turns the
@@ -40,16 +41,17 @@ namespace mdz {
 namespace {
 
 constexpr uint32_t kMinRun = 3, kMaxRun = 130, kMaxLit = 128;
-constexpr uint32_t kEncThreads = 1024, kEncWaves = kEncThreads / kWave;
 constexpr uint32_t kPer = 32;                   // bytes per thread and window
-constexpr uint32_t kWin = kEncThreads * kPer;
-constexpr uint32_t kStage = kWin + kWin / 32;   // staged output bytes of a window
 
+template <uint32_t kWaves>
 struct EncLds {
+    static constexpr uint32_t kThreads = kWaves * kWave;
+    static constexpr uint32_t kWin = kThreads * kPer;
+    static constexpr uint32_t kStage = kWin + kWin / 32 + 64;    // staged output bytes of a window
     alignas(16) uint32_t in[kWin / 4];
     alignas(16) uint32_t out[kStage / 4 + 8];
     uint16_t list[kWin];                        // window offsets where a segment ends
-    uint32_t part[3][kEncWaves];
+    uint32_t part[3][kWaves];
 };
 
 // Pending literals after a segment of L >= 3 bytes that starts as runs.
@@ -149,16 +151,17 @@ MDZ_DEV int32_t write_segment(Put put, int32_t o, uint32_t& n, uint32_t L, uint3
     return o;
 }
 
-// Exclusive scan over the workgroup through part[16]: `incl` is the wave's
+// Exclusive scan over the workgroup through part[kWaves]: `incl` is the wave's
 // inclusive scan, `carry` comes before the workgroup's first thread and takes
 // in its last.  One barrier; every row of 16 lanes then scans the parts.
-template <class Then>
+template <uint32_t kWaves, class Then>
 MDZ_DEV uint32_t block_scan(uint32_t* part, uint32_t incl, uint32_t& carry, Then then) {
-    static_assert(kEncWaves == 16, "the parts fill a row");
+    static_assert(kWaves <= 16, "the parts fit a row");
     const uint32_t wave = threadIdx.x / kWave;
     if (lane_id() == kWave - 1) part[wave] = incl;
     __syncthreads();
-    uint32_t v = part[lane_id() & 15];
+    const uint32_t w = lane_id() & 15;
+    uint32_t v = w < kWaves ? part[min(w, kWaves - 1)] : 0u;
     v = then(dpp_src<0x111, 0xf, 0u>(v), v);              // 0 is every map's identity
     v = then(dpp_src<0x112, 0xf, 0u>(v), v);
     v = then(dpp_src<0x114, 0xf, 0u>(v), v);
@@ -169,13 +172,12 @@ MDZ_DEV uint32_t block_scan(uint32_t* part, uint32_t incl, uint32_t& carry, Then
     return then(before, from_below(incl, 0));
 }
 
-__global__ __launch_bounds__(kEncThreads) void brle_encode_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes,
-                                                                  uint64_t chunk, uint64_t slot,
-                                                                  uint8_t* __restrict__ work,
-                                                                  uint64_t* __restrict__ sizes) {
-    __shared__ EncLds S;
+// One chunk c, by the whole workgroup.
+template <uint32_t kWaves>
+MDZ_DEV void encode_chunk(EncLds<kWaves>& S, uint64_t c, const uint8_t* __restrict__ in, uint64_t in_bytes,
+                          uint64_t chunk, uint64_t slot, uint8_t* __restrict__ work, uint64_t* __restrict__ sizes) {
+    constexpr uint32_t kEncThreads = EncLds<kWaves>::kThreads, kWin = EncLds<kWaves>::kWin, kStage = EncLds<kWaves>::kStage;
     const uint32_t t = threadIdx.x;
-    const uint64_t c = blockIdx.x;
     const uint64_t base = c * chunk;
     const uint32_t len = (uint32_t)min(chunk, in_bytes - base);
     const uint8_t* src = in + base;
@@ -235,7 +237,7 @@ __global__ __launch_bounds__(kEncThreads) void brle_encode_kernel(const uint8_t*
         uint32_t count = 0;
         {
             const uint32_t mine = (uint32_t)__builtin_popcount(ends);
-            uint32_t i = block_scan(S.part[0], wave_incl_scan_u32(mine), count, plus);
+            uint32_t i = block_scan<kWaves>(S.part[0], wave_incl_scan_u32(mine), count, plus);
             for (uint32_t m = ends; m; m &= m - 1) S.list[i++] = (uint16_t)(at + (uint32_t)__builtin_ctz(m));
         }
         __syncthreads();
@@ -251,12 +253,12 @@ __global__ __launch_bounds__(kEncThreads) void brle_encode_kernel(const uint8_t*
         // 2. literals pending before the thread's first segment
         uint32_t map = 0;
         each([&](uint32_t L, uint32_t) { map = map_then(map, map_of(L)); });
-        uint32_t n = map_apply(block_scan(S.part[1], wave_incl_maps(map), state, map_then), 0);
+        uint32_t n = map_apply(block_scan<kWaves>(S.part[1], wave_incl_maps(map), state, map_then), 0);
         // 3. where its bytes go
         uint32_t bytes = 0, n3 = n;
         each([&](uint32_t L, uint32_t) { bytes += count_segment(n3, L); });
         uint32_t total = 0;
-        const uint32_t off = block_scan(S.part[2], wave_incl_scan_u32(bytes), total, plus);
+        const uint32_t off = block_scan<kWaves>(S.part[2], wave_incl_scan_u32(bytes), total, plus);
         // 4. write them.  LDS byte i holds output byte (staged & ~15) + i; what
         // does not fit there (long runs), and headers stored before, go straight out
         const uint64_t stage0 = staged & ~15ull;
@@ -304,6 +306,19 @@ __global__ __launch_bounds__(kEncThreads) void brle_encode_kernel(const uint8_t*
         const int32_t o = write_segment(put, 0, n, len - open, last);
         if (n) put(o - 1 - (int32_t)n, n + 127);
         sizes[c] = done + (uint32_t)o;
+    }
+}
+
+// Chunks beyond the grid's workgroups are taken in turn.
+template <uint32_t kWaves>
+__global__ __launch_bounds__(kWaves * kWave) void brle_encode_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes,
+                                                                     uint64_t n_chunks, uint64_t chunk, uint64_t slot,
+                                                                     uint8_t* __restrict__ work,
+                                                                     uint64_t* __restrict__ sizes) {
+    __shared__ EncLds<kWaves> S;
+    for (uint64_t c = blockIdx.x; c < n_chunks; c += gridDim.x) {
+        encode_chunk<kWaves>(S, c, in, in_bytes, chunk, slot, work, sizes);
+        __syncthreads();
     }
 }
 
@@ -383,8 +398,11 @@ int brle_compress(const void* in, uint64_t in_bytes, uint64_t chunk, void* work,
     if (n > (1ull << 24)) return MDZ_ERR_INVALID;     // grid sizes stay below 2^32 threads
     const uint64_t slot = (wb - 8 * n) / n;
     uint64_t* sizes = reinterpret_cast<uint64_t*>(static_cast<uint8_t*>(work) + n * slot);
-    hipLaunchKernelGGL(brle_encode_kernel, dim3((uint32_t)n), dim3(kEncThreads), 0, s,
-                       static_cast<const uint8_t*>(in), in_bytes, chunk, slot, static_cast<uint8_t*>(work), sizes);
+    // a workgroup no wider than its chunk's windows: 2, 8 or 32 KiB
+    const uint32_t waves = chunk <= EncLds<1>::kWin ? 1 : chunk <= EncLds<4>::kWin ? 4 : 16;
+    auto encode = waves == 1 ? brle_encode_kernel<1> : waves == 4 ? brle_encode_kernel<4> : brle_encode_kernel<16>;
+    hipLaunchKernelGGL(encode, dim3((uint32_t)(n < (1u << 20) ? n : 1u << 20)), dim3(waves * kWave), 0, s,
+                       static_cast<const uint8_t*>(in), in_bytes, n, chunk, slot, static_cast<uint8_t*>(work), sizes);
     hipError_t e = hipGetLastError();
     if (e != hipSuccess) return record_hip(e, "brle_encode_kernel launch");
     hipLaunchKernelGGL(brle_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, sizes, n, ptr);

@@ -72,12 +72,12 @@ def _segments(size, lengths, seed):
 
 
 # segment lengths that meet the 128-literal and 130-run limits from every
-# phase; chunks around the 32 KiB window, of odd sizes (so chunks start at any
+# phase; chunks around the workgroups' windows (2, 8 and 32 KiB), of odd sizes (so chunks start at any
 # byte) and with runs longer than a window's staged output
 @pytest.mark.parametrize("lengths", [[1], [1, 2], [1, 2, 3], [1, 2, 125, 126, 127, 128, 129],
                                      [1, 3, 129, 130, 131, 132, 133, 259, 260, 261, 262, 263],
                                      [1, 2, 40_000], [1, 5_000_000]])
-@pytest.mark.parametrize("chunk", [1, 127, 1000, 32767, 32768, 32769, 65541, 262144, 9_000_000])
+@pytest.mark.parametrize("chunk", [1, 127, 1000, 2048, 2049, 8192, 8193, 32767, 32768, 32769, 65541, 262144, 9_000_000])
 def test_segment_lengths(gpu, lengths, chunk):
     from compression_amd import brle
     from compression_amd._lib import DeviceBuffer
@@ -93,3 +93,17 @@ def test_segment_lengths(gpu, lengths, chunk):
         got = ptr.download(8 * (n + 1)).view(np.uint64)
         assert np.array_equal(got, ref.ptr)
         assert dst.download(int(got[-1])).tobytes() == ref.data.tobytes()
+
+
+def test_more_chunks_than_workgroups(gpu):
+    from compression_amd import brle
+    from compression_amd._lib import DeviceBuffer
+    data = host.gen_brle_u8((1 << 20) * 2 + 7, 71)
+    n, wb, cap = brle.compress_bound(data.size, 2)
+    src, work, dst, ptr = DeviceBuffer.from_array(data), DeviceBuffer(wb), DeviceBuffer(cap), DeviceBuffer(8 * (n + 1))
+    print(f"brle encode {n} chunks of 2 bytes", flush=True)
+    brle.compress(src, data.size, dst, ptr, work, chunk_bytes=2)
+    ref = host.brle_encode(data, 2)
+    got = ptr.download(8 * (n + 1)).view(np.uint64)
+    assert n > 1 << 20 and np.array_equal(got, ref.ptr)
+    assert dst.download(int(got[-1])).tobytes() == ref.data.tobytes()
