@@ -72,7 +72,8 @@ hipError_t launch(const mdz_lanes_t& in, void* dst, uint64_t dst_bytes, int32_t*
     if (!quarters) {
         const size_t smem = (size_t)data_cap + 16 + sizeof(Rlev2Tables<PartPool<32>::value>);
         const uint64_t bytes = dst_bytes < in.chunk_bytes ? dst_bytes : in.chunk_bytes;
-        const bool wide = 2 * smem > kLdsPerCu && bytes / EB >= kWideValues;
+        // (a launch holds under 2^32 threads)
+        const bool wide = 2 * smem > kLdsPerCu && bytes / EB >= kWideValues && in.n_chunks < (1ull << 32) / kWideThreads;
         auto k = wide ? rlev2_decode_kernel<EB, kWideThreads> : rlev2_decode_kernel<EB, kThreads>;
         if ((e = set_dynamic_lds((const void*)k, smem)) != hipSuccess) return e;
         hipLaunchKernelGGL(k, dim3((uint32_t)in.n_chunks), dim3(wide ? kWideThreads : kThreads), smem, s, a);
