@@ -34,6 +34,7 @@
 // segments that end in its own bytes, 22.0 ms with one lane walking a chunk).
 // Groups go to a per-chunk slot of the work buffer; a scan kernel turns the
 // chunk sizes into ptr[] and a shift kernel packs the slots into `data`.
+#include "brle_load.h"
 #include "mdz_device.h"
 #include "mdz_internal.h"
 
@@ -41,7 +42,7 @@ namespace mdz {
 namespace {
 
 constexpr uint32_t kMinRun = 3, kMaxRun = 130, kMaxLit = 128;
-constexpr uint32_t kPer = 32;                   // bytes per thread and window
+constexpr uint32_t kPer = kBrlePer;             // bytes per thread and window
 
 template <uint32_t kWaves>
 struct EncLds {
@@ -202,7 +203,7 @@ MDZ_DEV void encode_chunk(EncLds<kWaves>& S, uint64_t c, const uint8_t* __restri
                 const uint4 q = p[i];
                 v[4 * i] = q.x, v[4 * i + 1] = q.y, v[4 * i + 2] = q.z, v[4 * i + 3] = q.w;
             }
-        } else if (w0 + at >= skew && w0 + at + kPer + 4 <= len) {
+        } else if (brle_whole_dwords(w0, at, len, skew)) {
             // whole dwords around the bytes, shifted together
             const uint32_t* p = reinterpret_cast<const uint32_t*>(src + w0 + at - skew);
             uint32_t lo = p[0];
