@@ -97,3 +97,29 @@ def test_token_limits(gpu, dtype, lane_values, line_values):
         assert np.array_equal(got, ref.blk_off), name
         assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len), name
         assert pay.download(int(got[-1])).tobytes() == ref.payload[:int(got[-1])].tobytes(), name
+
+
+# lane streams of 30 to 34 words, and empty-handed neighbours of 1 to 2: the
+# interleave stores chunks of at most 32 rounds without a tile
+@pytest.mark.parametrize("lane_values", [118, 122, 123, 126, 127, 131])
+def test_interleave_rounds(gpu, lane_values):
+    from compression_amd import rle_v1
+    from compression_amd._lib import DeviceBuffer
+    rng = np.random.default_rng(lane_values)
+    n_chunks, chunk = 9, 32 * lane_values
+    lanes = np.where(np.arange(lane_values) % 2, 100, 3).astype(np.uint8)   # literals of one byte each
+    data = np.zeros((n_chunks, lane_values, 32), np.uint8)                  # lines of one byte
+    for c in range(n_chunks):
+        full = rng.random(32) < c / (n_chunks - 1)
+        data[c][:, full] = lanes[:, None]
+    raw = data.reshape(-1)
+    n, wb, cap = rle_v1.compress_bound(raw.size, chunk, 1, 1)
+    src, work, pay = DeviceBuffer.from_array(raw), DeviceBuffer(wb), DeviceBuffer(cap)
+    col, off = DeviceBuffer(256 * n), DeviceBuffer(8 * (n + 1))
+    print(f"rlev1 encode interleave {lane_values} lane values n={n}", flush=True)
+    rle_v1.compress(src, raw.size, chunk, 1, 1, work, pay, col, off)
+    ref = host.rlev1_encode(raw, chunk, 1)
+    got = off.download(8 * (n + 1)).view(np.uint64)
+    assert np.array_equal(got, ref.blk_off)
+    assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len)
+    assert pay.download(int(got[-1])).tobytes() == ref.payload[:int(got[-1])].tobytes()
