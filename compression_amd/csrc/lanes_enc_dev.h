@@ -28,20 +28,48 @@ inline dim3 lane_grid(uint64_t n_chunks) {       // the kernels stride over the 
     return dim3((uint32_t)(u < (1u << 24) ? u : 1u << 24));
 }
 
-// chunk_len[c]: the chunk's lanes rounded up to words, their sum to 128
-// bytes.  Half a wave per chunk.
-constexpr uint32_t kSizeThreads = 256, kSizeChunks = kSizeThreads / 32;
+// Output of a lane stream that one thread encodes: stored by whole words, the
+// last up to three bytes held back.  The stream's slot has room for the last
+// word.
+struct WordOut {
+    uint8_t* out;
+    uint32_t len = 0, held = 0;
 
-__global__ __launch_bounds__(kSizeThreads) void lanes_size_kernel(const uint64_t* __restrict__ col_len, uint64_t n,
-                                                                  uint64_t* __restrict__ chunk_len) {
-    const uint64_t c = (uint64_t)blockIdx.x * kSizeChunks + threadIdx.x / 32;
-    const uint32_t words = c < n ? (uint32_t)((col_len[c * 32 + threadIdx.x % 32] + 3) / 4) : 0u;
+    MDZ_DEV void put(uint32_t b) {               // b < 256
+        held |= b << (8 * (len & 3));
+        if ((++len & 3) == 0) {
+            *reinterpret_cast<uint32_t*>(out + len - 4) = held;
+            held = 0;
+        }
+    }
+    MDZ_DEV void patch(uint32_t at, uint32_t b) {        // a byte put as 0
+        if (at >= (len & ~3u)) held |= b << (8 * (at & 3));
+        else out[at] = (uint8_t)b;
+    }
+    MDZ_DEV uint32_t finish() {                  // the stream's bytes
+        if (len & 3) *reinterpret_cast<uint32_t*>(out + (len & ~3u)) = held;
+        return len;
+    }
+};
+
+// chunk_len[c]: the chunk's lanes rounded up to words, their sum to 128
+// bytes.  Half a wave per chunk, a lane stream's words in each lane; all lanes
+// of the wave take part, whether c < n or not.
+MDZ_DEV void store_chunk_len(uint32_t words, uint64_t c, uint64_t n, uint64_t* __restrict__ chunk_len) {
     const uint32_t incl = wave_incl_scan_u32(words);
     const uint32_t low = (uint32_t)__builtin_amdgcn_readlane((int)incl, 31);
     if (c < n && threadIdx.x % 32 == 31) {
         const uint32_t total = lane_id() < 32 ? incl : incl - low;
         chunk_len[c] = ((uint64_t)total * 4 + 127) / 128 * 128;
     }
+}
+
+constexpr uint32_t kSizeThreads = 256, kSizeChunks = kSizeThreads / 32;
+
+__global__ __launch_bounds__(kSizeThreads) void lanes_size_kernel(const uint64_t* __restrict__ col_len, uint64_t n,
+                                                                  uint64_t* __restrict__ chunk_len) {
+    const uint64_t c = (uint64_t)blockIdx.x * kSizeChunks + threadIdx.x / 32;
+    store_chunk_len(c < n ? (uint32_t)((col_len[c * 32 + threadIdx.x % 32] + 3) / 4) : 0u, c, n, chunk_len);
 }
 
 constexpr uint32_t kScanThreads = 1024;

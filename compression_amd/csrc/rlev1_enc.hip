@@ -19,7 +19,8 @@
 //      an LDS stage.  A header whose count is not known yet (a group or run
 //      that goes on past the window) is written when it closes.  64 MiB of
 //      4-byte values in 128 KiB chunks: 106 us, vector and scalar issue about
-//      equal (1030 us with one lane encoding each stream).
+//      equal (1030 us with one lane encoding each stream).  Streams of a few
+//      values are encoded by a thread each.
 //   2. Small kernels sum the rounded lane lengths per chunk and scan them into
 //      blk_off.
 //   3. The lane streams are interleaved in the round-robin order of
@@ -79,6 +80,34 @@ MDZ_DEV uint32_t step_code(typename Wide<EB>::T x, typename Wide<EB>::T prev) {
     return fits ? 0x100u | ((uint32_t)d & 0xFFu) : 0u;
 }
 
+// Values of lane t of chunk c: byte k*EB of the lane sits in line t + 32*(k*EB
+// / line).  A chunk inside the input, aligned, with lines of a power of two:
+// one load a value.
+template <int EB>
+struct LaneValues {
+    typedef typename Wide<EB>::T T;
+    typedef typename std::conditional<EB == 8, uint64_t, typename std::conditional<EB == 4, uint32_t,
+            typename std::conditional<EB == 2, uint16_t, uint8_t>::type>::type>::type Elem;
+    const uint8_t *in, *src;
+    uint64_t in_bytes, base;
+    uint32_t n, line, t, shift;
+    bool plain;
+
+    MDZ_DEV LaneValues(const uint8_t* in_, uint64_t in_bytes_, uint64_t c, uint64_t chunk, uint32_t line_, uint32_t t_)
+        : in(in_), src(in_ + c * chunk), in_bytes(in_bytes_), base(c * chunk), n((uint32_t)(chunk / 32 / EB)),
+          line(line_), t(t_), shift(31 - __builtin_clz(line_)),
+          plain((line_ & (line_ - 1)) == 0 && (c + 1) * chunk <= in_bytes_ && ((uintptr_t)src & (EB - 1)) == 0) {}
+    MDZ_DEV T operator()(uint32_t k) const {     // any value past the last
+        if (plain) {
+            const uint32_t o = min(k, n - 1) * EB;
+            return *reinterpret_cast<const Elem*>(src + ((((uint64_t)(o >> shift) * 32 + t) << shift) | (o & (line - 1))));
+        }
+        if (k >= n) return 0;
+        const uint32_t o = k * EB, r = o / line, j = o - r * line;
+        return (T)load_elem(in, in_bytes, base + (t + 32ull * r) * line + j, EB);
+    }
+};
+
 template <class T>
 MDZ_DEV uint32_t leb_bytes(T v) {                // ceil(bits / 7), at least 1
     const uint32_t bits = sizeof(T) == 8 ? 64 - (uint32_t)__builtin_clzll((uint64_t)v | 1) : 32 - (uint32_t)__builtin_clz((uint32_t)v | 1);
@@ -118,29 +147,13 @@ __global__ __launch_bounds__(kWave) void rlev1_encode_kernel(const uint8_t* __re
                                                              uint64_t lane_slot, uint8_t* __restrict__ work,
                                                              uint64_t* __restrict__ col_len) {
     typedef typename Wide<EB>::T T;
-    typedef typename std::conditional<EB == 8, uint64_t, typename std::conditional<EB == 4, uint32_t,
-            typename std::conditional<EB == 2, uint16_t, uint8_t>::type>::type>::type Elem;
     __shared__ uint32_t stage[kStageBytes / 4 + 1];
     const uint32_t l = lane_id(), n = (uint32_t)(chunk / 32 / EB);
-    const bool pow2 = (line & (line - 1)) == 0;
-    const uint32_t shift = 31 - __builtin_clz(line);
     for (uint64_t unit = blockIdx.x; unit < lane_units(n_chunks); unit += gridDim.x) {
         uint64_t c;
         uint32_t t;
         if (!lane_of_unit(unit, n_chunks, c, t)) continue;
-        // lane value k: byte k*EB sits in line t + 32*(k*EB / line).  A chunk
-        // inside the input, aligned, with lines of a power of two: one load.
-        const uint8_t* src = in + c * chunk;
-        const bool plain = pow2 && (c + 1) * chunk <= in_bytes && ((uintptr_t)src & (EB - 1)) == 0;
-        auto value = [&](uint32_t k) -> T {
-            if (plain) {
-                const uint32_t o = min(k, n - 1) * EB;
-                return *reinterpret_cast<const Elem*>(src + ((((uint64_t)(o >> shift) * 32 + t) << shift) | (o & (line - 1))));
-            }
-            if (k >= n) return 0;
-            const uint32_t o = k * EB, r = o / line, j = o - r * line;
-            return (T)load_elem(in, in_bytes, c * chunk + (t + 32ull * r) * line + j, EB);
-        };
+        const LaneValues<EB> value(in, in_bytes, c, chunk, line, t);
         LaneStage w{reinterpret_cast<uint8_t*>(stage), work + (c * 32 + t) * lane_slot, 0, 0};
         uint32_t lit = 0, lit_at = 0;            // open literal group: values so far, header's offset
         uint32_t ones = 0, run_at = 0;           // open run: bits of S so far, count byte's offset
@@ -248,6 +261,80 @@ __global__ __launch_bounds__(kWave) void rlev1_encode_kernel(const uint8_t* __re
     }
 }
 
+// Short lane streams: a thread encodes one, value by value, half a wave per
+// chunk.  No group or run of so few values is full.  A window of 64 values
+// costs a wave the same whatever it holds: 65536 chunks of 2 4-byte values a
+// lane take 811 us with a wave per stream and 34 us so, 3276 of 40 values 48 and
+// 40 us.  One thread's values wait for each other, though: few chunks leave the
+// chip empty either way, and there a wave is the faster from about 9 values a
+// lane on (512 chunks of 16: 17 us a call against 19; 2048 chunks: 38 against 23).
+constexpr uint32_t kShortThreads = 256, kShortChunks = kShortThreads / 32;
+constexpr uint32_t kShortValues = 8, kShortOfMany = 40, kManyChunks = 2048;
+static_assert(kShortOfMany <= kMaxGroup && kShortOfMany <= kMaxRunLen, "short streams fill no token");
+inline bool short_lanes(uint64_t values, uint64_t n_chunks) {
+    return values <= kShortValues || (values <= kShortOfMany && n_chunks >= kManyChunks);
+}
+
+template <int EB>
+__global__ __launch_bounds__(kShortThreads) void rlev1_short_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes,
+                                                                    uint64_t n_chunks, uint64_t chunk, uint32_t line,
+                                                                    uint64_t lane_slot, uint8_t* __restrict__ work,
+                                                                    uint64_t* __restrict__ col_len,
+                                                                    uint64_t* __restrict__ chunk_len) {
+    typedef typename Wide<EB>::T T;
+    const uint64_t c = (uint64_t)blockIdx.x * kShortChunks + threadIdx.x / 32;
+    const uint32_t t = threadIdx.x % 32, n = (uint32_t)(chunk / 32 / EB);
+    uint32_t len = 0;
+    if (c < n_chunks) {
+        const LaneValues<EB> value(in, in_bytes, c, chunk, line, t);
+        WordOut o{work + (c * 32 + t) * lane_slot};
+        uint32_t lit = 0, lit_at = 0;            // open literal group: values so far, header's offset
+        auto varint = [&](T v) {
+            for (; v > 0x7F; v >>= 7) o.put(((uint32_t)v & 0x7Fu) | 0x80u);
+            o.put((uint32_t)v);
+        };
+        // x0, x1: the first value not yet written and its successor; s: x1's step code
+        T x0 = value(0), x1 = value(1);
+        uint32_t s = step_code<EB>(x1, x0), p = 0;
+        while (p < n) {
+            T x2 = value(p + 2);
+            uint32_t s2 = p + 2 < n ? step_code<EB>(x2, x1) : 0;
+            if (s && s2 == s) {
+                if (lit) o.patch(lit_at, 256 - lit);
+                lit = 0;
+                uint32_t m = 2;
+                do {                             // x2 is value p + m, in the run
+                    ++m;
+                    x1 = x2;
+                    x2 = value(p + m);
+                    s2 = p + m < n ? step_code<EB>(x2, x1) : 0;
+                } while (s2 == s);
+                o.put(m - kMinRunLen);
+                o.put(s & 0xFFu);
+                varint(x0);
+                p += m;
+                x0 = x2;
+                x1 = value(p + 1);
+                s = p + 1 < n ? step_code<EB>(x1, x0) : 0;
+            } else {
+                if (lit++ == 0) {
+                    lit_at = o.len;
+                    o.put(0);
+                }
+                varint(x0);
+                ++p;
+                x0 = x1;
+                x1 = x2;
+                s = s2;
+            }
+        }
+        if (lit) o.patch(lit_at, 256 - lit);
+        len = o.finish();
+        col_len[c * 32 + t] = len;
+    }
+    store_chunk_len((len + 3) / 4, c, n_chunks, chunk_len);
+}
+
 uint64_t lane_slot_bytes(uint64_t chunk, uint32_t eb) {
     const uint64_t n = chunk / 32 / eb;
     return (n * 11 + 16 + 15) & ~15ull;          // LEB128 <= 10 bytes per value, plus headers
@@ -276,15 +363,24 @@ int rlev1_compress(const void* in, uint64_t in_bytes, uint64_t chunk, uint32_t e
     if (!in || !work || !payload || !col_len || !blk_off || n > (1ull << 24)) return MDZ_ERR_INVALID;
     const uint64_t slot = lane_slot_bytes(chunk, eb);
     uint64_t* chunk_len = reinterpret_cast<uint64_t*>(static_cast<uint8_t*>(work) + n * 32 * slot);
-    auto encode = eb == 1 ? rlev1_encode_kernel<1> : eb == 2 ? rlev1_encode_kernel<2>
-                : eb == 4 ? rlev1_encode_kernel<4> : rlev1_encode_kernel<8>;
-    hipLaunchKernelGGL(encode, lane_grid(n), dim3(kWave), 0, s, static_cast<const uint8_t*>(in), in_bytes, n, chunk,
-                       line, slot, static_cast<uint8_t*>(work), col_len);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return record_hip(e, "rlev1_encode_kernel launch");
-    hipLaunchKernelGGL(lanes_size_kernel, dim3((uint32_t)((n + kSizeChunks - 1) / kSizeChunks)), dim3(kSizeThreads), 0, s,
-                       col_len, n, chunk_len);
-    if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lanes_size_kernel launch");
+    hipError_t e;
+    if (short_lanes(chunk / 32 / eb, n)) {
+        auto encode = eb == 1 ? rlev1_short_kernel<1> : eb == 2 ? rlev1_short_kernel<2>
+                    : eb == 4 ? rlev1_short_kernel<4> : rlev1_short_kernel<8>;
+        hipLaunchKernelGGL(encode, dim3((uint32_t)((n + kShortChunks - 1) / kShortChunks)), dim3(kShortThreads), 0, s,
+                           static_cast<const uint8_t*>(in), in_bytes, n, chunk, line, slot,
+                           static_cast<uint8_t*>(work), col_len, chunk_len);
+        if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "rlev1_short_kernel launch");
+    } else {
+        auto encode = eb == 1 ? rlev1_encode_kernel<1> : eb == 2 ? rlev1_encode_kernel<2>
+                    : eb == 4 ? rlev1_encode_kernel<4> : rlev1_encode_kernel<8>;
+        hipLaunchKernelGGL(encode, lane_grid(n), dim3(kWave), 0, s, static_cast<const uint8_t*>(in), in_bytes, n,
+                           chunk, line, slot, static_cast<uint8_t*>(work), col_len);
+        if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "rlev1_encode_kernel launch");
+        hipLaunchKernelGGL(lanes_size_kernel, dim3((uint32_t)((n + kSizeChunks - 1) / kSizeChunks)), dim3(kSizeThreads),
+                           0, s, col_len, n, chunk_len);
+        if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lanes_size_kernel launch");
+    }
     hipLaunchKernelGGL(lanes_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, chunk_len, n, blk_off, nullptr, ~0ull);
     if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lanes_scan_kernel launch");
     hipLaunchKernelGGL(lanes_interleave_kernel, interleave_grid(n, slot), dim3(kIlvThreads), 0, s,

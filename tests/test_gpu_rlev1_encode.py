@@ -123,3 +123,35 @@ def test_interleave_rounds(gpu, lane_values):
     assert np.array_equal(got, ref.blk_off)
     assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len)
     assert pay.download(int(got[-1])).tobytes() == ref.payload[:int(got[-1])].tobytes()
+
+
+# both forms of the encoder: a thread per lane stream up to 8 values, and up to
+# 40 where there are 2048 chunks or more; a wave per stream beyond
+@pytest.mark.parametrize("dtype", [np.uint32, np.uint64, np.uint16, np.uint8])
+@pytest.mark.parametrize("lane_values,n_chunks", [(2, 3), (5, 9), (8, 8), (9, 8), (9, 2047), (9, 2048), (40, 2047),
+                                                  (40, 2049), (41, 2048)])
+def test_short_lanes(gpu, dtype, lane_values, n_chunks):
+    from compression_amd import rle_v1
+    from compression_amd._lib import DeviceBuffer
+    eb = np.dtype(dtype).itemsize
+    chunk, nvals = 32 * lane_values * eb, 32 * lane_values * n_chunks - 3
+    rng = np.random.default_rng(lane_values + n_chunks + eb)
+    steps = np.repeat(rng.choice(np.array([-129, -128, -3, 0, 1, 127, 128, 1 << 20]), nvals // 2 + 1), 2)
+    steps[rng.random(steps.size) < 0.2] = 0
+    # lane t's values are t, t + 32, ...: make each lane's neighbours meet
+    walk = np.cumsum(steps[:nvals]).astype(np.int64)
+    walk = np.concatenate([walk, np.zeros(3, np.int64)]).reshape(n_chunks, 32, lane_values).swapaxes(1, 2).reshape(-1)
+    for name, x in {"walk": walk.view(np.uint64)[:nvals], "wide": rng.integers(0, 2**64, nvals, dtype=np.uint64),
+                    "bits": rng.integers(0, 2, nvals).astype(np.uint64)}.items():
+        data = x.astype(dtype)
+        raw = data.view(np.uint8)
+        n, wb, cap = rle_v1.compress_bound(raw.size, chunk, eb, eb)
+        src, work, pay = DeviceBuffer.from_array(raw), DeviceBuffer(wb), DeviceBuffer(cap)
+        col, off = DeviceBuffer(256 * n), DeviceBuffer(8 * (n + 1))
+        print(f"rlev1 encode {name} {eb} bytes, {lane_values} lane values n={n}", flush=True)
+        rle_v1.compress(src, raw.size, chunk, eb, eb, work, pay, col, off)
+        ref = host.rlev1_encode(data, chunk, eb)
+        got = off.download(8 * (n + 1)).view(np.uint64)
+        assert n == n_chunks and np.array_equal(got, ref.blk_off), name
+        assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len), name
+        assert pay.download(int(got[-1])).tobytes() == ref.payload[:int(got[-1])].tobytes(), name
