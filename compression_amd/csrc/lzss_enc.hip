@@ -24,7 +24,8 @@
 // per stream up to 2048 lane bytes (64 KiB chunks), 14 KiB beyond.  Lanes over
 // 4096 bytes are indexed in windows of 4096 positions that advance by 2048.
 // 64 MiB in 64 KiB chunks: 2.7 ms (3.4 ms with one position a step; 412 ms with
-// one lane per stream and chains in global memory).
+// one lane per stream and chains in global memory).  Streams of a few bytes are
+// encoded by a thread each.
 //
 // A second kernel ranks a chunk's 32 lanes by length (descending, ties to
 // the higher lane id) into col_map; the shared kernels scan the chunk
@@ -257,7 +258,22 @@ __global__ __launch_bounds__(kWave) void lzss_encode_kernel(const uint8_t* __res
 }
 
 // Sorted slot of lane t: longer lanes first, equal lengths by higher lane id.
-// Half a wave per chunk.
+// Half a wave per chunk, `len` its lane lengths (the caller's own at len[t]).
+MDZ_DEV void rank_lanes(const uint32_t* len, uint32_t t, uint64_t c, uint64_t n_chunks, uint64_t* __restrict__ col_len,
+                        uint8_t* __restrict__ col_map, uint64_t* __restrict__ chunk_len) {
+    const uint32_t mine = len[t];
+    uint32_t rank = 0, words = 0;
+    for (uint32_t u = 0; u < kHalf; ++u) {
+        const uint32_t other = len[u];
+        rank += (other > mine || (other == mine && u > t)) ? 1u : 0u;
+        words += (other + 3) / 4;
+    }
+    if (c >= n_chunks) return;
+    col_len[c * 32 + rank] = mine;
+    col_map[c * 32 + rank] = (uint8_t)t;
+    if (t == 0) chunk_len[c] = ((uint64_t)words * 4 + 127) / 128 * 128;
+}
+
 constexpr uint32_t kRankThreads = 256, kRankChunks = kRankThreads / kHalf;
 
 __global__ __launch_bounds__(kRankThreads) void lzss_rank_kernel(const uint32_t* __restrict__ lane_len, uint64_t n_chunks,
@@ -267,19 +283,92 @@ __global__ __launch_bounds__(kRankThreads) void lzss_rank_kernel(const uint32_t*
     __shared__ uint32_t len[kRankThreads];
     const uint32_t t = threadIdx.x % kHalf;
     const uint64_t c = (uint64_t)blockIdx.x * kRankChunks + threadIdx.x / kHalf;
-    const uint32_t mine = c < n_chunks ? lane_len[c * 32 + t] : 0u;
-    len[threadIdx.x] = mine;
+    len[threadIdx.x] = c < n_chunks ? lane_len[c * 32 + t] : 0u;
     wave_sync();
-    uint32_t rank = 0, words = 0;
-    for (uint32_t u = 0; u < kHalf; ++u) {
-        const uint32_t other = len[threadIdx.x - t + u];
-        rank += (other > mine || (other == mine && u > t)) ? 1u : 0u;
-        words += (other + 3) / 4;
+    rank_lanes(len + (threadIdx.x - t), t, c, n_chunks, col_len, col_map, chunk_len);
+}
+
+// Short lane streams: a thread encodes one, its bytes in a column of LDS, half a
+// wave per chunk; every earlier position is a candidate.  An index costs a wave
+// the same however few positions it holds: 131072 chunks of 4 bytes a lane take
+// 1810 us with a wave per stream and 56 us so, 16384 chunks of 32 bytes 950 and
+// 130 us (Markov text).  A thread's time grows with the square of its bytes
+// (129 us at 32) and few chunks do not fill the chip, so the more bytes the more
+// chunks it takes: 1024 chunks of 32 bytes take 72 us a call with a wave per
+// stream, 129 us so.  8 bytes take 12 us however few chunks there are, 14 us
+// with a wave.
+constexpr uint32_t kShortBytes = 8, kShortOfMany = 64, kShortChunks = kWave / kHalf;
+inline bool short_lanes(uint32_t bytes, uint64_t n_chunks) {
+    return bytes <= kShortBytes || (bytes <= kShortOfMany && n_chunks >= 2ull * bytes * bytes);
+}
+
+__global__ __launch_bounds__(kWave) void lzss_short_kernel(const uint8_t* __restrict__ in, uint64_t n_chunks,
+                                                           uint64_t chunk, uint64_t lane_slot,
+                                                           uint8_t* __restrict__ work, uint64_t* __restrict__ col_len,
+                                                           uint8_t* __restrict__ col_map,
+                                                           uint64_t* __restrict__ chunk_len) {
+    __shared__ uint32_t data[kShortOfMany / 4 + 1][kWave];        // the last row is read, not used
+    __shared__ uint32_t len[kWave];
+    const uint32_t l = lane_id(), t = l % kHalf, n = (uint32_t)(chunk / 32);
+    const uint64_t c = (uint64_t)blockIdx.x * kShortChunks + l / kHalf;
+    uint32_t bytes = 0;
+    if (c < n_chunks) {
+        const uint8_t* rows = in + c * chunk + 4 * t;
+        for (uint32_t k = 0; k < n / 4; ++k) data[k][l] = *reinterpret_cast<const uint32_t*>(rows + 128ull * k);
+        auto at = [&](uint32_t p) { return alignbyte(data[p / 4 + 1][l], data[p / 4][l], p & 3); };   // 4 bytes
+        WordOut o{work + (c * 32 + t) * lane_slot};
+        o.put(0);
+        uint32_t flag_at = 0, ntok = 0, flags = 0;
+        for (uint32_t cur = 0; cur < n;) {
+            const uint32_t here = at(cur);
+            uint32_t best = kMinLen - 1, from = 0;
+            // candidates four at a time, oldest first; position 0 is none, nor
+            // one too near for a longer match
+            const uint32_t most = min(n - cur, kMaxLen);
+            uint32_t lo = data[0][l];
+            for (uint32_t q4 = 0; q4 + best < cur && best < most; q4 += 4) {
+                const uint32_t hi = data[q4 / 4 + 1][l];
+                const uint32_t x0 = q4 ? (lo ^ here) << 8 : 1u, x1 = (alignbyte(hi, lo, 1) ^ here) << 8,
+                               x2 = (alignbyte(hi, lo, 2) ^ here) << 8, x3 = (alignbyte(hi, lo, 3) ^ here) << 8;
+                lo = hi;
+                if (min(min(x0, x1), min(x2, x3))) continue;     // no 3 equal bytes
+                for (uint32_t j = 0; j < 4; ++j) {
+                    if (j == 0 ? x0 : j == 1 ? x1 : j == 2 ? x2 : x3) continue;
+                    const uint32_t q = q4 + j, cap = q < cur ? min(cur - q, most) : 0u;
+                    uint32_t f = 0;
+                    while (f < cap) {
+                        const uint32_t x = at(q + f) ^ at(cur + f);
+                        f += x ? (uint32_t)__builtin_ctz(x) >> 3 : 4u;
+                        if (x) break;
+                    }
+                    f = min(f, cap);
+                    if (f > best) best = f, from = q;
+                }
+            }
+            if (best < kMinLen) {
+                flags |= 1u << ntok;
+                o.put(here & 0xFFu);
+                cur += 1;
+            } else {
+                const uint32_t v = (cur - from) << kLenBits | (best - kMinLen);
+                o.put(v & 0xFFu);
+                o.put(v >> 8);
+                cur += best;
+            }
+            if (++ntok == 8) {                  // the next group's flag byte is reserved at once
+                o.patch(flag_at, flags);
+                flags = 0;
+                ntok = 0;
+                flag_at = o.len;
+                o.put(0);
+            }
+        }
+        o.patch(flag_at, flags);
+        bytes = o.finish();
     }
-    if (c >= n_chunks) return;
-    col_len[c * 32 + rank] = mine;
-    col_map[c * 32 + rank] = (uint8_t)t;
-    if (t == 0) chunk_len[c] = ((uint64_t)words * 4 + 127) / 128 * 128;
+    len[l] = bytes;
+    wave_sync();
+    rank_lanes(len + (l - t), t, c, n_chunks, col_len, col_map, chunk_len);
 }
 
 uint64_t lz_lane_slot(uint64_t chunk) {
@@ -316,14 +405,20 @@ int lzss_compress(const void* in, uint64_t in_bytes, uint64_t chunk, void* work,
     uint32_t* lane_len = reinterpret_cast<uint32_t*>(w + n * 32 * slot);
     uint64_t* chunk_len = reinterpret_cast<uint64_t*>(w + n * 32 * slot + n * chunk * 2);
     const uint32_t lb = (uint32_t)(chunk / 32);
-    const dim3 grid = lane_grid(n), block(kWave);
-    auto encode = lb <= 1024 ? lzss_encode_kernel<1024> : lb <= 2048 ? lzss_encode_kernel<2048> : lzss_encode_kernel<4096>;
-    hipLaunchKernelGGL(encode, grid, block, 0, s, static_cast<const uint8_t*>(in), n, chunk, slot, w, lane_len);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return record_hip(e, "lzss_encode_kernel launch");
-    hipLaunchKernelGGL(lzss_rank_kernel, dim3((uint32_t)((n + kRankChunks - 1) / kRankChunks)), dim3(kRankThreads), 0, s,
-                       lane_len, n, col_len, col_map, chunk_len);
-    if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lzss_rank_kernel launch");
+    hipError_t e;
+    if (short_lanes(lb, n)) {
+        hipLaunchKernelGGL(lzss_short_kernel, dim3((uint32_t)((n + kShortChunks - 1) / kShortChunks)), dim3(kWave), 0, s,
+                           static_cast<const uint8_t*>(in), n, chunk, slot, w, col_len, col_map, chunk_len);
+        if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lzss_short_kernel launch");
+    } else {
+        auto encode = lb <= 1024 ? lzss_encode_kernel<1024> : lb <= 2048 ? lzss_encode_kernel<2048> : lzss_encode_kernel<4096>;
+        hipLaunchKernelGGL(encode, lane_grid(n), dim3(kWave), 0, s, static_cast<const uint8_t*>(in), n, chunk, slot, w,
+                           lane_len);
+        if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lzss_encode_kernel launch");
+        hipLaunchKernelGGL(lzss_rank_kernel, dim3((uint32_t)((n + kRankChunks - 1) / kRankChunks)), dim3(kRankThreads), 0,
+                           s, lane_len, n, col_len, col_map, chunk_len);
+        if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lzss_rank_kernel launch");
+    }
     hipLaunchKernelGGL(lanes_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, chunk_len, n, blk_off, nullptr, ~0ull);
     if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lanes_scan_kernel launch");
     hipLaunchKernelGGL(lanes_interleave_kernel, interleave_grid(n, slot), dim3(kIlvThreads), 0, s,

@@ -74,3 +74,29 @@ def test_window_edges(gpu, lane_bytes):
         assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len), name
         assert np.array_equal(cmap.download(32 * n), ref.col_map), name
         assert pay.download(int(ref.blk_off[-1])).tobytes() == ref.payload[:int(ref.blk_off[-1])].tobytes(), name
+
+
+# both forms of the encoder: a thread per lane stream up to 8 bytes, and up to
+# 64 where there are at least 2 * bytes * bytes chunks; a wave per stream beyond
+@pytest.mark.parametrize("lane_bytes,n_chunks", [(4, 3), (8, 7), (12, 7), (12, 287), (12, 288), (32, 2047), (32, 2049),
+                                                 (64, 8191), (64, 8193), (68, 9248)])
+def test_short_lanes(gpu, lane_bytes, n_chunks):
+    from compression_amd import lzss
+    from compression_amd._lib import DeviceBuffer
+    chunk = 32 * lane_bytes
+    size = n_chunks * chunk
+    rng = np.random.default_rng(lane_bytes + n_chunks)
+    kinds = {"markov": host.gen_lzss_markov(size, lane_bytes), "pairs": rng.integers(0, 2, size).astype(np.uint8),
+             "mixed": np.where(rng.random(size) < 0.1, rng.integers(0, 256, size), 7).astype(np.uint8),
+             "random": rng.integers(0, 256, size).astype(np.uint8), "zeros": np.zeros(size, np.uint8)}
+    for name, data in kinds.items():
+        n, wb, cap = lzss.compress_bound(size, chunk)
+        src, work, pay = DeviceBuffer.from_array(data), DeviceBuffer(wb), DeviceBuffer(cap)
+        col, cmap, off = DeviceBuffer(256 * n), DeviceBuffer(32 * n), DeviceBuffer(8 * (n + 1))
+        print(f"lzss encode {name} lane_bytes={lane_bytes} n={n}", flush=True)
+        lzss.compress(src, size, chunk, work, pay, col, cmap, off)
+        ref = host.lzss_encode(data, chunk)
+        assert np.array_equal(off.download(8 * (n + 1)).view(np.uint64), ref.blk_off), name
+        assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len), name
+        assert np.array_equal(cmap.download(32 * n), ref.col_map), name
+        assert pay.download(int(ref.blk_off[-1])).tobytes() == ref.payload[:int(ref.blk_off[-1])].tobytes(), name
