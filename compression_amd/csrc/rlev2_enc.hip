@@ -437,6 +437,194 @@ __global__ __launch_bounds__(kWave) void rlev2_encode_kernel(const uint8_t* __re
     }
 }
 
+// Short lane streams: a thread encodes one, value by value, its values in a
+// column of LDS, half a wave per chunk.  No group of so few values is full.  A
+// group costs a wave the same however few values it holds: 131072 chunks of 1
+// 8-byte value a lane take 2700 us with a wave per stream and 107 us so, 8192
+// chunks of 16 values 231 and 165 us (the benchmark's column; constant values
+// 143 and 13 us).  A thread's time grows with its values and few chunks do not
+// fill the chip, so the more values the more chunks it takes: 256 chunks of 16
+// 8-byte values take 22 us a call with a wave per stream and 127 us so.  Three
+// values take 11 us however few chunks there are, 14 us with a wave.  Beyond 16
+// values the benchmark's column is slower with a thread (24: 300 against 165
+// us), bytes beyond 32 (48: 273 against 174 us).
+constexpr uint32_t kShortValues = 3, kShortOfMany = 16, kShortBytesOfMany = 32, kShortChunks = kWave / 32;
+static_assert(kShortBytesOfMany < kMaxLit, "short streams fill no group");
+inline bool short_lanes(uint64_t values, uint32_t eb, uint64_t n_chunks) {
+    return values <= kShortValues ||
+           (values <= (eb == 1 ? kShortBytesOfMany : kShortOfMany) && n_chunks >= 192 * values);
+}
+
+// One thread's lane stream: values val[0..nv), strided by a wave, and output.
+template <class LT>
+struct ShortLane {
+    const LT* val;
+    WordOut o;
+    uint32_t cur = 0, fill = 0;                  // bits of the byte being packed
+
+    MDZ_DEV uint64_t at(uint32_t i) const { return val[i * kWave]; }
+    MDZ_DEV void byte(uint64_t v) { o.put((uint32_t)v & 0xFFu); }
+    // The low w bits of v, most significant first.
+    MDZ_DEV void field(uint64_t v, uint32_t w) {
+        while (w) {
+            const uint32_t take = min(w, 8 - fill);
+            w -= take;
+            cur = cur << take | ((uint32_t)(v >> w) & ((1u << take) - 1u));
+            if ((fill += take) == 8) pad();
+        }
+    }
+    MDZ_DEV void pad() {
+        if (fill) byte(cur << (8 - fill));
+        cur = 0;
+        fill = 0;
+    }
+    MDZ_DEV void bytes(uint64_t v, uint32_t count) {
+        while (count) byte(v >> (8 * --count));
+    }
+    MDZ_DEV void varint(uint64_t v) {
+        for (; v > 0x7F; v >>= 7) byte((v & 0x7F) | 0x80);
+        byte(v);
+    }
+    // header, first value and zigzag step of a delta group
+    MDZ_DEV void delta_head(uint32_t code, uint64_t first, uint64_t step, uint32_t n) {
+        bytes(header(0xC0, code, n), 2);
+        varint(first);
+        varint((step << 1) ^ (uint64_t)((int64_t)step >> 63));
+    }
+    MDZ_DEV void run(uint64_t v, uint32_t n) {
+        if (n > kMaxShortRepeat) return delta_head(0, v, 0, n);
+        const uint32_t vbytes = (value_width(v) - 1) / 8 + 1;
+        byte(((vbytes - 1) << 3) | (n - kMinRepeat));
+        bytes(v, vbytes);
+    }
+    MDZ_DEV void direct(uint32_t s, uint32_t n, uint64_t all) {          // all: the values' bits
+        const uint32_t w = aligned_width(value_width(all));
+        bytes(header(0x40, width_code(w), n), 2);
+        for (uint32_t i = 0; i < n; ++i) field(at(s + i), w);
+        pad();
+    }
+    // How many of the offsets from base have a width code of at least c.
+    MDZ_DEV uint32_t at_least(uint32_t s, uint32_t n, uint64_t base, uint32_t c) const {
+        uint32_t k = 0;
+        for (uint32_t i = 0; i < n; ++i) k += width_code(bit_length(at(s + i) - base)) >= c ? 1u : 0u;
+        return k;
+    }
+    MDZ_DEV void patched(uint32_t s, uint32_t n, uint64_t base, uint32_t b95, uint32_t b100) {
+        uint32_t pw = fixed_width(b100 - b95);
+        if (pw == 64) {
+            pw = 56;
+            b95 = 8;
+        }
+        const uint64_t mask = (1ull << b95) - 1;
+        uint32_t np = 0, prev = 0, max_gap = 0;
+        for (uint32_t i = 0; i < n; ++i) {
+            if (at(s + i) - base > mask) {
+                max_gap = max(max_gap, i - prev);
+                prev = i;
+                ++np;
+            }
+        }
+        const uint32_t pgw = value_width(max_gap), vbytes = value_width(base) / 8 + 1;
+        bytes(header(0x80, width_code(b95), n), 2);
+        bytes((((vbytes - 1) << 5) | width_code(pw)) << 8 | ((((pgw - 1) << 5) | np) & 0xFF), 2);
+        if (vbytes > 8) byte(0);
+        bytes(base, min(vbytes, 8u));
+        for (uint32_t i = 0; i < n; ++i) field((at(s + i) - base) & mask, fixed_width(b95));
+        pad();
+        prev = 0;
+        for (uint32_t i = 0; i < n; ++i) {
+            const uint64_t r = at(s + i) - base;
+            if (r > mask) {
+                field((uint64_t)(i - prev) << pw | r >> b95, fixed_width(pgw + pw));
+                prev = i;
+            }
+        }
+        pad();
+    }
+    // The rules of literals() above for values [s, s + n).
+    MDZ_DEV void literals(uint32_t s, uint32_t n) {
+        const uint64_t first = at(s), step = n > 1 ? at(s + 1) - first : 0;
+        uint64_t all = first, low = first, high = first, steps = 0, p = first;
+        bool even = true, up = true, down = true;
+        for (uint32_t i = 1; i < n; ++i) {
+            const uint64_t v = at(s + i);
+            all |= v;
+            low = min(low, v);
+            high = max(high, v);
+            steps |= v - p;
+            even = even && v - p == step;
+            up = up && p <= v;
+            down = down && p >= v;
+            p = v;
+        }
+        if (n <= kMinRepeat || (low == 0 && high <= 128)) return direct(s, n, all);
+        if (even) return delta_head(0, first, step, n);
+        if (step && (up || down)) {
+            const uint32_t w = max(2u, aligned_width(value_width(steps)));
+            delta_head(width_code(w), first, step, n);
+            for (uint32_t i = 2; i < n; ++i) field(at(s + i) - at(s + i - 1), w);
+            return pad();
+        }
+        const uint32_t code = width_code(bit_length(all)), near = code < 24 ? max(code, 1u) - 1 : code;
+        if (at_least(s, n, 0, near) <= (n * 10 - 1) / 100 + 1) {
+            const uint32_t c100 = width_code(bit_length(high - low)), above = (n * 5 - 1) / 100 + 1;
+            if (at_least(s, n, low, c100) <= above) {
+                uint32_t c95 = 0;
+                for (uint32_t bit = 16; bit; bit >>= 1)
+                    if (at_least(s, n, low, c95 | bit) > above) c95 |= bit;
+                return patched(s, n, low, code_width(c95), code_width(c100));
+            }
+        }
+        direct(s, n, all);
+    }
+    MDZ_DEV uint32_t encode(uint32_t nv) {       // the stream's bytes
+        for (uint32_t s = 0; s < nv;) {
+            const uint64_t v = at(s);
+            uint32_t n = 1;
+            while (s + n < nv && at(s + n) == v) ++n;
+            if (n >= kMinRepeat) {
+                run(v, n);
+            } else {                             // up to the first three equal values in a row
+                uint32_t same = n;
+                uint64_t p = v;
+                for (; s + n < nv && same < kMinRepeat; ++n) {
+                    const uint64_t x = at(s + n);
+                    same = x == p ? same + 1 : 1;
+                    p = x;
+                }
+                if (same == kMinRepeat) n -= kMinRepeat;
+                literals(s, n);
+            }
+            s += n;
+        }
+        return o.finish();
+    }
+};
+
+template <int EB>
+__global__ __launch_bounds__(kWave) void rlev2_short_kernel(const uint8_t* __restrict__ in, uint64_t in_bytes,
+                                                            uint64_t n_chunks, uint64_t chunk, uint32_t ru,
+                                                            uint64_t lane_slot, uint8_t* __restrict__ work,
+                                                            uint64_t* __restrict__ col_len,
+                                                            uint64_t* __restrict__ chunk_len) {
+    typedef typename std::conditional<EB == 8, uint64_t, uint32_t>::type LT;
+    extern __shared__ __align__(8) uint8_t short_vals[];         // nv values per thread
+    LT* val = reinterpret_cast<LT*>(short_vals);
+    const uint32_t l = lane_id(), t = l % 32, nv = (uint32_t)(chunk / EB / 32);
+    const uint64_t c = (uint64_t)blockIdx.x * kShortChunks + l / 32;
+    uint32_t len = 0;
+    if (c < n_chunks) {
+        for (uint32_t q = 0, line = 0, at = 0; q < nv; ++q) {
+            val[q * kWave + l] = (LT)chunk_value(in, in_bytes, c * chunk, ((uint64_t)line * 32 + t) * ru + at, EB);
+            if (++at == ru) at = 0, ++line;
+        }
+        ShortLane<LT> e{val + l, WordOut{work + (c * 32 + t) * lane_slot}};
+        len = e.encode(nv);
+        col_len[c * 32 + t] = len;
+    }
+    store_chunk_len((len + 3) / 4, c, n_chunks, chunk_len);
+}
+
 uint64_t v2_lane_slot(uint64_t chunk, uint32_t eb) {
     return (chunk / eb / 32 * 10 + 64 + 15) & ~15ull;
 }
@@ -464,16 +652,24 @@ int rlev2_compress(const void* in, uint64_t in_bytes, uint64_t chunk, uint32_t e
     if (!in || !work || !payload || !col_len || !blk_off || n > (1ull << 24)) return MDZ_ERR_INVALID;
     const uint64_t slot = v2_lane_slot(chunk, eb);
     uint64_t* chunk_len = reinterpret_cast<uint64_t*>(static_cast<uint8_t*>(work) + n * 32 * slot);
-    const dim3 grid = lane_grid(n), block(kWave);
-    auto encode = eb == 1 ? rlev2_encode_kernel<1> : eb == 2 ? rlev2_encode_kernel<2>
-                : eb == 4 ? rlev2_encode_kernel<4> : rlev2_encode_kernel<8>;
-    hipLaunchKernelGGL(encode, grid, block, 0, s, static_cast<const uint8_t*>(in), in_bytes, n, chunk, ru, slot,
-                       static_cast<uint8_t*>(work), col_len);
-    hipError_t e = hipGetLastError();
-    if (e != hipSuccess) return record_hip(e, "rlev2_encode_kernel launch");
-    hipLaunchKernelGGL(lanes_size_kernel, dim3((uint32_t)((n + kSizeChunks - 1) / kSizeChunks)), dim3(kSizeThreads), 0, s,
-                       col_len, n, chunk_len);
-    if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lanes_size_kernel launch");
+    hipError_t e;
+    if (short_lanes(chunk / eb / 32, eb, n)) {
+        auto encode = eb == 1 ? rlev2_short_kernel<1> : eb == 2 ? rlev2_short_kernel<2>
+                    : eb == 4 ? rlev2_short_kernel<4> : rlev2_short_kernel<8>;
+        hipLaunchKernelGGL(encode, dim3((uint32_t)((n + kShortChunks - 1) / kShortChunks)), dim3(kWave),
+                           chunk / eb / 32 * kWave * (eb == 8 ? 8 : 4), s, static_cast<const uint8_t*>(in), in_bytes, n,
+                           chunk, ru, slot, static_cast<uint8_t*>(work), col_len, chunk_len);
+        if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "rlev2_short_kernel launch");
+    } else {
+        auto encode = eb == 1 ? rlev2_encode_kernel<1> : eb == 2 ? rlev2_encode_kernel<2>
+                    : eb == 4 ? rlev2_encode_kernel<4> : rlev2_encode_kernel<8>;
+        hipLaunchKernelGGL(encode, lane_grid(n), dim3(kWave), 0, s, static_cast<const uint8_t*>(in), in_bytes, n, chunk,
+                           ru, slot, static_cast<uint8_t*>(work), col_len);
+        if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "rlev2_encode_kernel launch");
+        hipLaunchKernelGGL(lanes_size_kernel, dim3((uint32_t)((n + kSizeChunks - 1) / kSizeChunks)), dim3(kSizeThreads),
+                           0, s, col_len, n, chunk_len);
+        if ((e = hipGetLastError()) != hipSuccess) return record_hip(e, "lanes_size_kernel launch");
+    }
     // blk_off[n] holds the uncompressed size; the true payload end goes to *payload_bytes
     hipLaunchKernelGGL(lanes_scan_kernel, dim3(1), dim3(kScanThreads), 0, s, chunk_len, n, blk_off, payload_bytes,
                        in_bytes);

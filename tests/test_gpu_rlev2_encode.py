@@ -117,3 +117,37 @@ def test_group_limits(gpu, dtype, lane_values, ru):
         nbytes = int(pb.download(8).view(np.uint64)[0])
         assert nbytes == ref.payload_bytes, name
         assert pay.download(nbytes).tobytes() == ref.payload[:nbytes].tobytes(), name
+
+
+# both forms of the encoder: a thread per lane stream up to 3 values, and up to
+# 16 (bytes: 32) where there are 192 chunks or more per value; a wave beyond
+@pytest.mark.parametrize("dtype", [np.uint64, np.uint32, np.uint16, np.uint8])
+@pytest.mark.parametrize("lane_values,n_chunks", [(1, 5), (2, 5), (3, 5), (4, 767), (4, 769), (9, 1728), (16, 3071),
+                                                  (16, 3073), (17, 3265), (32, 6145), (33, 6336)])
+def test_short_lanes(gpu, dtype, lane_values, n_chunks):
+    from compression_amd import rlev2
+    from compression_amd._lib import DeviceBuffer
+    eb = np.dtype(dtype).itemsize
+    chunk, nvals = 32 * lane_values * eb, 32 * lane_values * n_chunks - 5
+    rng = np.random.default_rng(lane_values + n_chunks + eb)
+    m = nvals + 5
+    kinds = dict(_shapes(m, lane_values + eb))
+    kinds["outliers"] = np.where(rng.random(m) < 0.08, rng.integers(2**30, 2**64, m, dtype=np.uint64),
+                                 rng.integers(1, 2**int(rng.integers(1, 20)), m).astype(np.uint64))
+    kinds["repeats"] = np.repeat(rng.integers(0, 2**50, m), rng.integers(1, 14, m))[:m].astype(np.uint64)
+    for name, x in kinds.items():
+        # lane t's values are t, t + 32, ...: make neighbours of x one lane's
+        x = x.reshape(n_chunks, 32, lane_values).swapaxes(1, 2).reshape(-1)[:nvals]
+        data = (x >> np.uint64(0 if eb == 8 else 5)).astype(dtype)
+        raw = data.view(np.uint8)
+        n, wb, cap = rlev2.compress_bound(raw.size, chunk, eb, 1)
+        src, work, pay, pb = DeviceBuffer.from_array(raw), DeviceBuffer(wb), DeviceBuffer(cap), DeviceBuffer(8)
+        col, off = DeviceBuffer(256 * n), DeviceBuffer(8 * (n + 1))
+        print(f"rlev2 encode {name} {eb} bytes, {lane_values} lane values n={n}", flush=True)
+        rlev2.compress(src, raw.size, chunk, eb, 1, work, pay, col, off, pb)
+        ref = host.rlev2_encode(data, chunk, 1)
+        assert n == n_chunks and np.array_equal(off.download(8 * (n + 1)).view(np.uint64), ref.blk_off), name
+        assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len), name
+        nbytes = int(pb.download(8).view(np.uint64)[0])
+        assert nbytes == ref.payload_bytes, name
+        assert pay.download(nbytes).tobytes() == ref.payload[:nbytes].tobytes(), name
