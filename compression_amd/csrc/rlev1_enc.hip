@@ -268,11 +268,14 @@ __global__ __launch_bounds__(kWave) void rlev1_encode_kernel(const uint8_t* __re
 // 40 us.  One thread's values wait for each other, though: few chunks leave the
 // chip empty either way, and there a wave is the faster from about 9 values a
 // lane on (512 chunks of 16: 17 us a call against 19; 2048 chunks: 38 against 23).
+// Bytes stay faster with a thread up to a whole window (4096 chunks of 64: 69 us
+// against 98), wider values do not (2048 chunks of 64 8-byte values: 73 against 65).
 constexpr uint32_t kShortThreads = 256, kShortChunks = kShortThreads / 32;
-constexpr uint32_t kShortValues = 8, kShortOfMany = 40, kManyChunks = 2048;
-static_assert(kShortOfMany <= kMaxGroup && kShortOfMany <= kMaxRunLen, "short streams fill no token");
-inline bool short_lanes(uint64_t values, uint64_t n_chunks) {
-    return values <= kShortValues || (values <= kShortOfMany && n_chunks >= kManyChunks);
+constexpr uint32_t kShortValues = 8, kShortOfMany = 40, kShortBytesOfMany = 64, kManyChunks = 2048;
+static_assert(kShortBytesOfMany <= kMaxGroup && kShortBytesOfMany <= kMaxRunLen, "short streams fill no token");
+inline bool short_lanes(uint64_t values, uint32_t eb, uint64_t n_chunks) {
+    return values <= kShortValues ||
+           (values <= (eb == 1 ? kShortBytesOfMany : kShortOfMany) && n_chunks >= kManyChunks);
 }
 
 template <int EB>
@@ -364,7 +367,7 @@ int rlev1_compress(const void* in, uint64_t in_bytes, uint64_t chunk, uint32_t e
     const uint64_t slot = lane_slot_bytes(chunk, eb);
     uint64_t* chunk_len = reinterpret_cast<uint64_t*>(static_cast<uint8_t*>(work) + n * 32 * slot);
     hipError_t e;
-    if (short_lanes(chunk / 32 / eb, n)) {
+    if (short_lanes(chunk / 32 / eb, eb, n)) {
         auto encode = eb == 1 ? rlev1_short_kernel<1> : eb == 2 ? rlev1_short_kernel<2>
                     : eb == 4 ? rlev1_short_kernel<4> : rlev1_short_kernel<8>;
         hipLaunchKernelGGL(encode, dim3((uint32_t)((n + kShortChunks - 1) / kShortChunks)), dim3(kShortThreads), 0, s,

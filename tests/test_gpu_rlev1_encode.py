@@ -126,10 +126,10 @@ def test_interleave_rounds(gpu, lane_values):
 
 
 # both forms of the encoder: a thread per lane stream up to 8 values, and up to
-# 40 where there are 2048 chunks or more; a wave per stream beyond
+# 40 (bytes: 64) where there are 2048 chunks or more; a wave per stream beyond
 @pytest.mark.parametrize("dtype", [np.uint32, np.uint64, np.uint16, np.uint8])
 @pytest.mark.parametrize("lane_values,n_chunks", [(2, 3), (5, 9), (8, 8), (9, 8), (9, 2047), (9, 2048), (40, 2047),
-                                                  (40, 2049), (41, 2048)])
+                                                  (40, 2049), (41, 2048), (64, 2048), (65, 2048)])
 def test_short_lanes(gpu, dtype, lane_values, n_chunks):
     from compression_amd import rle_v1
     from compression_amd._lib import DeviceBuffer
