@@ -27,7 +27,9 @@ constexpr uint32_t kQuarterLanes = 8, kQuarterThreads = 256;
 // that 8 did.  Three 128 KiB chunks of 8-byte values 42.7 -> 33.7 us, 64 MiB of
 // 4-byte values 169 -> 129 us, of bytes 469 -> 357 us.  A chunk of few values
 // has too few runs for them: 2048 of 8 bytes take 21.8 us with 512 threads and
-// 23.1 with 1024, 3072 take 25.4 and 24.1.
+// 23.1 with 1024, 3072 take 25.4 and 24.1; 3072 of 1, 2 and 4 bytes 21.9, 21.7
+// and 21.3 with 512, 20.2, 21.0 and 20.6 with 1024.  Chunks of that many values
+// and few runs (equal values, 40 equal in a row, ramps, random) gain or stay.
 constexpr uint32_t kWideThreads = 1024, kLdsPerCu = 160 * 1024, kWideValues = 3072;
 
 template <int EB, uint32_t NT>

@@ -442,7 +442,8 @@ struct Rlev2Tables {
     uint32_t fits;
     uint32_t extent_ok;
     uint32_t pub;            // records the walk has published this epoch
-    uint32_t claimed;        // records claimed by consumer waves (windows of Rlev2Args::win)
+    uint32_t claimed;        // records claimed by consumer waves (windows of Rlev2Args::win); claims
+                             // where windows differ in length
     uint32_t final_;         // records of this epoch once the walk has ended, else kOpen
     uint32_t more;           // a lane stream has runs left after this epoch
     uint32_t total;          // words of all lanes
@@ -484,6 +485,12 @@ template <int EB, uint32_t NL, uint32_t NT>
 MDZ_DEV void rlev2_part(const Rlev2Args& a, uint64_t c, uint32_t part, uint32_t* smem) {
     static_assert(NL >= 1 && NL <= 32 && 32 % NL == 0 && NT % kWave == 0 && NT >= 128, "part shape");
     constexpr uint32_t kRunPool = PartPool<NL>::value;
+    // In a workgroup wider than kThreads the first windows, one per wave, are half
+    // as long: chunks of few long runs then occupy all waves.  Three chunks of
+    // 128 runs (128 KiB of equal 8-byte values) take 16.2 us, 21.3 us with 8 of
+    // the 16 waves at work (19.0 us in 512 threads); of 256 runs 25.9 us, 23.3 us
+    // with whole windows (29.1 us); the benchmark's column 32.3 us either way.
+    constexpr uint32_t kHalves = NT > kThreads ? NT / kWave : 0;
     typedef Rlev2Tables<kRunPool> Tables;
     constexpr uint64_t vmask = EB == 8 ? ~0ull : ((1ull << (8 * EB)) - 1);
     const uint8_t* __restrict__ payload = a.payload;
@@ -590,21 +597,26 @@ MDZ_DEV void rlev2_part(const Rlev2Args& a, uint64_t c, uint32_t part, uint32_t*
             MDZ_PHASE(2);
         }
         for (;;) {
-            uint32_t w0 = 0;
-            if (l == 0) w0 = atomicAdd(&tb.claimed, win);
+            uint32_t w0 = 0, size = win;
+            if (l == 0) w0 = atomicAdd(&tb.claimed, kHalves ? 1u : win);
             w0 = __builtin_amdgcn_readfirstlane(w0);
+            if constexpr (kHalves != 0) {           // claims are counted, not records
+                const uint32_t half = win / 2, k = w0;
+                size = k < kHalves ? half : win;
+                w0 = k < kHalves ? k * half : kHalves * half + (k - kHalves) * win;
+            }
             uint32_t avail = 0;
             for (uint32_t it = 0;; ++it) {
                 const uint32_t fin = __hip_atomic_load(&tb.final_, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
                 if (fin != kOpen) { avail = fin; break; }
                 const uint32_t pv = __hip_atomic_load(&tb.pub, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_WORKGROUP);
-                if (pv >= w0 + win) { avail = w0 + win; break; }
+                if (pv >= w0 + size) { avail = w0 + size; break; }
                 if (it >= kSpinMax) { if (l == 0) tb.stuck = 1; break; }
                 __builtin_amdgcn_s_sleep(2);
             }
             avail = __builtin_amdgcn_readfirstlane(avail);
             if (w0 >= avail) break;
-            const uint32_t cnt = min(win, avail - w0);
+            const uint32_t cnt = min(size, avail - w0);
             // check, one record per lane: the oracle's checks in its order
             // (patch lists included) complete the descriptor in registers,
             // and the run's parameters are decoded here, one run per lane

@@ -155,3 +155,19 @@ def test_workgroup_widths(gpu, dtype, nvals, max_chunk):
     print(f"rlev2 decode {nvals} values of {eb} bytes, max_chunk {max_chunk}", flush=True)
     got, st = _run(gpu, c, max_chunk=max_chunk)
     assert (st == 0).all() and np.array_equal(got, x.view(np.uint8))
+
+
+# 1024-thread workgroups: each wave's first window is half as long; few and many
+# runs against every window length
+@pytest.mark.parametrize("window", [0, 8, 16, 32, 64])
+@pytest.mark.parametrize("kind", ["one", "few", "ramp", "many"])
+@pytest.mark.parametrize("dtype", [np.uint64, np.uint8])
+def test_wide_windows(gpu, dtype, kind, window):
+    eb = np.dtype(dtype).itemsize
+    n = 16384 * 2 + 77
+    x = {"one": np.full(n, 5), "few": np.repeat(np.arange(n // 1000 + 1), 1000)[:n], "ramp": np.arange(n) * 3,
+         "many": np.repeat(np.arange(n // 4 + 1), 4)[:n]}[kind].astype(dtype)
+    c = O.rlev2_encode(x, 16384 * eb, 64, threads=4)
+    print(f"rlev2 decode {kind} {eb} bytes, window {window}", flush=True)
+    got, st = _run(gpu, c, window=window)
+    assert (st == 0).all() and np.array_equal(got, x.view(np.uint8))
