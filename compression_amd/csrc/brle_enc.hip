@@ -395,8 +395,7 @@ int brle_compress(const void* in, uint64_t in_bytes, uint64_t chunk, void* work,
     uint64_t n = 0, wb = 0;
     int rc = brle_compress_bound(in_bytes, chunk, &n, &wb, nullptr);
     if (rc) return rc;
-    if (!in || !work || !data || !ptr) return MDZ_ERR_INVALID;
-    if (n > (1ull << 24)) return MDZ_ERR_INVALID;     // grid sizes stay below 2^32 threads
+    if (!in || !work || !data || !ptr || n > kMaxEncodeChunks) return MDZ_ERR_INVALID;
     const uint64_t slot = (wb - 8 * n) / n;
     uint64_t* sizes = reinterpret_cast<uint64_t*>(static_cast<uint8_t*>(work) + n * slot);
     // a workgroup no wider than its chunk's windows: 2, 8 or 32 KiB

@@ -398,7 +398,7 @@ int lzss_compress(const void* in, uint64_t in_bytes, uint64_t chunk, void* work,
     uint64_t n = 0;
     int rc = lzss_compress_bound(in_bytes, chunk, &n, nullptr, nullptr);
     if (rc) return rc;
-    if (!in || !work || !payload || !col_len || !col_map || !blk_off || n > (1ull << 24)) return MDZ_ERR_INVALID;
+    if (!in || !work || !payload || !col_len || !col_map || !blk_off || n > kMaxEncodeChunks) return MDZ_ERR_INVALID;
     if ((uintptr_t)in & 3) return MDZ_ERR_INVALID;   // lanes are read a dword at a time
     const uint64_t slot = lz_lane_slot(chunk);
     uint8_t* w = static_cast<uint8_t*>(work);

@@ -9,6 +9,10 @@
 
 namespace mdz {
 
+// Chunks an encoder takes: its launches of 256 threads a chunk stay below the
+// 2^32 threads that HIP refuses.
+constexpr uint64_t kMaxEncodeChunks = (1ull << 24) - 1;
+
 // Records a failed HIP call for mdz_last_error(); returns MDZ_OK/MDZ_ERR_HIP.
 int record_hip(hipError_t e, const char* what);
 // Formats a message for mdz_last_error() and returns rc.

@@ -649,7 +649,7 @@ int rlev2_compress(const void* in, uint64_t in_bytes, uint64_t chunk, uint32_t e
     uint64_t n = 0;
     int rc = rlev2_compress_bound(in_bytes, chunk, eb, ru, &n, nullptr, nullptr);
     if (rc) return rc;
-    if (!in || !work || !payload || !col_len || !blk_off || n > (1ull << 24)) return MDZ_ERR_INVALID;
+    if (!in || !work || !payload || !col_len || !blk_off || n > kMaxEncodeChunks) return MDZ_ERR_INVALID;
     const uint64_t slot = v2_lane_slot(chunk, eb);
     uint64_t* chunk_len = reinterpret_cast<uint64_t*>(static_cast<uint8_t*>(work) + n * 32 * slot);
     hipError_t e;

@@ -75,3 +75,15 @@ def test_encoder_bounds_checked_on_host():
     for chunk in (100, 2 << 20):
         assert lib.mdz_lzss_compress_bound(1 << 22, chunk, C.byref(n), C.byref(w), C.byref(p)) == -1
     assert lib.mdz_lzss_compress_bound(1000, 65536, C.byref(n), C.byref(w), C.byref(p)) == -1
+
+
+def test_encoders_refuse_too_many_chunks_on_host():
+    """2^24 chunks would pass HIP's limit of 2^32 - 1 threads a launch: refused
+    before the first of an encoder's kernels.  The pointers are never used."""
+    import compression_amd._lib as L
+    lib = L.lib()
+    n, p = 1 << 24, 4096
+    assert lib.mdz_rlev1_compress(p, 64 * n, 64, 1, 1, p, p, p, p, None) == -1
+    assert lib.mdz_rlev2_compress(p, 32 * n, 32, 1, 1, p, p, p, p, p, None) == -1
+    assert lib.mdz_brle_compress(p, n, 1, p, p, p, None) == -1
+    assert lib.mdz_lzss_compress(p, 128 * n, 128, p, p, p, p, p, None) == -1
