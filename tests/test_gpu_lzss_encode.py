@@ -100,3 +100,27 @@ def test_short_lanes(gpu, lane_bytes, n_chunks):
         assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len), name
         assert np.array_equal(cmap.download(32 * n), ref.col_map), name
         assert pay.download(int(ref.blk_off[-1])).tobytes() == ref.payload[:int(ref.blk_off[-1])].tobytes(), name
+
+
+def test_more_streams_than_workgroups(gpu):
+    """The wave form strides over its lane streams beyond 2^24 workgroups
+    (524,288 chunks): a period of 7 chunks, repeated, against the period's own
+    encoding."""
+    from compression_amd import lzss
+    from compression_amd._lib import DeviceBuffer
+    chunk, periods = 32 * 68, 524_288 // 7 + 2
+    one = host.gen_lzss_markov(7 * chunk, 23)
+    data = np.tile(one, periods)
+    n, wb, cap = lzss.compress_bound(data.size, chunk)
+    src, work, pay = DeviceBuffer.from_array(data), DeviceBuffer(wb), DeviceBuffer(cap)
+    col, cmap, off = DeviceBuffer(256 * n), DeviceBuffer(32 * n), DeviceBuffer(8 * (n + 1))
+    print(f"lzss encode {n} chunks", flush=True)
+    lzss.compress(src, data.size, chunk, work, pay, col, cmap, off)
+    ref = host.lzss_encode(one, chunk)
+    got, size = off.download(8 * (n + 1)).view(np.uint64), int(ref.blk_off[7])
+    assert n == 7 * periods > 524_288
+    assert np.array_equal(got[:-1].reshape(periods, 7),
+                          ref.blk_off[:7] + np.uint64(size) * np.arange(periods, dtype=np.uint64)[:, None])
+    assert (col.download(256 * n).view(np.uint64).reshape(periods, -1) == ref.col_len).all()
+    assert (cmap.download(32 * n).reshape(periods, -1) == ref.col_map).all()
+    assert (pay.download(size * periods).reshape(periods, -1) == ref.payload[:size]).all()

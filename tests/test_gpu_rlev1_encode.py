@@ -155,3 +155,50 @@ def test_short_lanes(gpu, dtype, lane_values, n_chunks):
         assert n == n_chunks and np.array_equal(got, ref.blk_off), name
         assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len), name
         assert pay.download(int(got[-1])).tobytes() == ref.payload[:int(got[-1])].tobytes(), name
+
+
+def test_more_streams_than_workgroups(gpu):
+    """The wave form strides over its lane streams beyond 2^24 workgroups
+    (524,288 chunks): a period of 7 chunks, repeated, against the period's own
+    encoding."""
+    from compression_amd import rle_v1
+    from compression_amd._lib import DeviceBuffer
+    lane_values, periods = 65, 524_288 // 7 + 2
+    chunk = 32 * lane_values
+    rng = np.random.default_rng(17)
+    one = np.where(rng.random(7 * chunk) < 0.6, 3, rng.integers(0, 256, 7 * chunk)).astype(np.uint8)
+    data = np.tile(one, periods)
+    n, wb, cap = rle_v1.compress_bound(data.size, chunk, 1, 1)
+    src, work, pay = DeviceBuffer.from_array(data), DeviceBuffer(wb), DeviceBuffer(cap)
+    col, off = DeviceBuffer(256 * n), DeviceBuffer(8 * (n + 1))
+    print(f"rlev1 encode {n} chunks", flush=True)
+    rle_v1.compress(src, data.size, chunk, 1, 1, work, pay, col, off)
+    ref = host.rlev1_encode(one, chunk, 1)
+    got, size = off.download(8 * (n + 1)).view(np.uint64), int(ref.blk_off[7])
+    assert n == 7 * periods > 524_288
+    assert np.array_equal(got[:-1].reshape(periods, 7),
+                          ref.blk_off[:7] + np.uint64(size) * np.arange(periods, dtype=np.uint64)[:, None])
+    assert (col.download(256 * n).view(np.uint64).reshape(periods, -1) == ref.col_len).all()
+    assert (pay.download(size * periods).reshape(periods, -1) == ref.payload[:size]).all()
+
+
+# inputs that start between elements, in both forms (5 and 130 lane values)
+@pytest.mark.parametrize("dtype,skip", [(np.uint16, 1), (np.uint32, 1), (np.uint32, 2), (np.uint64, 3), (np.uint64, 4)])
+@pytest.mark.parametrize("lane_values", [5, 130])
+def test_unaligned_input(gpu, dtype, skip, lane_values):
+    from compression_amd import rle_v1
+    from compression_amd._lib import DeviceBuffer
+    eb = np.dtype(dtype).itemsize
+    chunk = 32 * lane_values * eb
+    raw = host.gen_rlev1_u32(32 * lane_values * 7, lane_values).astype(dtype).view(np.uint8)
+    data = np.frombuffer(raw[skip:skip + (raw.size - skip) // eb * eb].tobytes(), dtype)
+    n, wb, cap = rle_v1.compress_bound(data.nbytes, chunk, eb, eb)
+    src, work, pay = DeviceBuffer.from_array(raw), DeviceBuffer(wb), DeviceBuffer(cap)
+    col, off = DeviceBuffer(256 * n), DeviceBuffer(8 * (n + 1))
+    print(f"rlev1 encode unaligned {eb} bytes skip {skip}", flush=True)
+    rle_v1.compress(src.ptr + skip, data.nbytes, chunk, eb, eb, work, pay, col, off)
+    ref = host.rlev1_encode(data, chunk, eb)
+    got = off.download(8 * (n + 1)).view(np.uint64)
+    assert np.array_equal(got, ref.blk_off)
+    assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len)
+    assert pay.download(int(got[-1])).tobytes() == ref.payload[:int(got[-1])].tobytes()

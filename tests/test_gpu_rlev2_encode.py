@@ -151,3 +151,50 @@ def test_short_lanes(gpu, dtype, lane_values, n_chunks):
         nbytes = int(pb.download(8).view(np.uint64)[0])
         assert nbytes == ref.payload_bytes, name
         assert pay.download(nbytes).tobytes() == ref.payload[:nbytes].tobytes(), name
+
+
+def test_more_streams_than_workgroups(gpu):
+    """The wave form strides over its lane streams beyond 2^24 workgroups
+    (524,288 chunks): a period of 7 chunks, repeated, against the period's own
+    encoding."""
+    from compression_amd import rlev2
+    from compression_amd._lib import DeviceBuffer
+    lane_values, periods = 33, 524_288 // 7 + 2
+    chunk = 32 * lane_values
+    one = _shapes(7 * chunk, 19)["mix"].astype(np.uint8)
+    data = np.tile(one, periods)
+    n, wb, cap = rlev2.compress_bound(data.size, chunk, 1, 1)
+    src, work, pay, pb = DeviceBuffer.from_array(data), DeviceBuffer(wb), DeviceBuffer(cap), DeviceBuffer(8)
+    col, off = DeviceBuffer(256 * n), DeviceBuffer(8 * (n + 1))
+    print(f"rlev2 encode {n} chunks", flush=True)
+    rlev2.compress(src, data.size, chunk, 1, 1, work, pay, col, off, pb)
+    ref = host.rlev2_encode(one, chunk, 1)
+    got, size = off.download(8 * (n + 1)).view(np.uint64), int(ref.payload_bytes)
+    assert n == 7 * periods > 524_288 and got[-1] == data.size
+    assert int(pb.download(8).view(np.uint64)[0]) == size * periods
+    assert np.array_equal(got[:-1].reshape(periods, 7),
+                          ref.blk_off[:7] + np.uint64(size) * np.arange(periods, dtype=np.uint64)[:, None])
+    assert (col.download(256 * n).view(np.uint64).reshape(periods, -1) == ref.col_len).all()
+    assert (pay.download(size * periods).reshape(periods, -1) == ref.payload[:size]).all()
+
+
+# inputs that start between elements, in both forms (3 and 130 lane values)
+@pytest.mark.parametrize("dtype,skip", [(np.uint16, 1), (np.uint32, 1), (np.uint32, 2), (np.uint64, 3), (np.uint64, 4)])
+@pytest.mark.parametrize("lane_values", [3, 130])
+def test_unaligned_input(gpu, dtype, skip, lane_values):
+    from compression_amd import rlev2
+    from compression_amd._lib import DeviceBuffer
+    eb = np.dtype(dtype).itemsize
+    chunk = 32 * lane_values * eb
+    raw = _shapes(32 * lane_values * 7, lane_values)["mix"].astype(dtype).view(np.uint8)
+    data = np.frombuffer(raw[skip:skip + (raw.size - skip) // eb * eb].tobytes(), dtype)
+    n, wb, cap = rlev2.compress_bound(data.nbytes, chunk, eb, 1)
+    src, work, pay, pb = DeviceBuffer.from_array(raw), DeviceBuffer(wb), DeviceBuffer(cap), DeviceBuffer(8)
+    col, off = DeviceBuffer(256 * n), DeviceBuffer(8 * (n + 1))
+    print(f"rlev2 encode unaligned {eb} bytes skip {skip}", flush=True)
+    rlev2.compress(src.ptr + skip, data.nbytes, chunk, eb, 1, work, pay, col, off, pb)
+    ref = host.rlev2_encode(data, chunk, 1)
+    assert np.array_equal(off.download(8 * (n + 1)).view(np.uint64), ref.blk_off)
+    assert np.array_equal(col.download(256 * n).view(np.uint64), ref.col_len)
+    nbytes = int(pb.download(8).view(np.uint64)[0])
+    assert nbytes == ref.payload_bytes and pay.download(nbytes).tobytes() == ref.payload[:nbytes].tobytes()
