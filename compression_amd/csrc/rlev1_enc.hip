@@ -18,7 +18,7 @@
 //      headers; a prefix sum over the lanes' byte counts places their bytes in
 //      an LDS stage.  A header whose count is not known yet (a group or run
 //      that goes on past the window) is written when it closes.  64 MiB of
-//      4-byte values in 128 KiB chunks: 106 us, vector and scalar issue about
+//      4-byte values in 128 KiB chunks: 95 us, vector and scalar issue about
 //      equal (1030 us with one lane encoding each stream).  Streams of a few
 //      values are encoded by a thread each.
 //   2. Small kernels sum the rounded lane lengths per chunk and scan them into

@@ -24,7 +24,7 @@ constexpr uint32_t kQuarterLanes = 8, kQuarterThreads = 256;
 // Where one workgroup's LDS leaves no room for a second on the CU (the caller
 // did not say how large a chunk is, or chunks are large), the workgroup is as
 // wide as the hardware allows: 16 waves stage the payload and decode the runs
-// that 8 did.  Three 128 KiB chunks of 8-byte values 42.7 -> 33.7 us, 64 MiB of
+// that 8 did.  Three 128 KiB chunks of 8-byte values 45 -> 32 us, 64 MiB of
 // 4-byte values 169 -> 129 us, of bytes 469 -> 357 us.  A chunk of few values
 // has too few runs for them: 2048 of 8 bytes take 21.8 us with 512 threads and
 // 23.1 with 1024, 3072 take 25.4 and 24.1; 3072 of 1, 2 and 4 bytes 21.9, 21.7

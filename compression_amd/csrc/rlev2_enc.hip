@@ -17,14 +17,17 @@
 //     inside the group, at most 128.
 // So per group the 64 lanes hold 128 values, two each, ballots of the equal
 // neighbours give the group, and the sub-mode is chosen from ballots and
-// counts (percentiles by a search over the width codes, five counts each).
-// Every writer packs most significant bit first, so all of them put fields at
-// bit positions: the lanes or their fields into an LDS stage of big-endian
-// words, which goes out in whole words.  A group costs about 300 instructions
-// instead of its values' serial chain.  256 MiB of 8-byte values in 128 KiB
-// chunks: 0.42 ms, bound by the groups' dependent ballots and LDS steps at 20
-// waves a CU (24.3 ms with one lane encoding each stream).  The scan and the
-// interleave are the shared lane-encoder kernels (lanes_enc_dev.h).
+// counts: the 90th and 95th percentile tests take one count each, of the values
+// that reach the next smaller width or the largest; only a patched group
+// searches the width codes for its percentile, five counts.  Every writer packs
+// most significant bit first, so all of them put fields at bit positions: the
+// lanes or their fields into an LDS stage of big-endian words, which goes out
+// in whole words.  A group costs about 300 instructions instead of its values'
+// serial chain.  256 MiB of 8-byte values in 128 KiB chunks: 0.30 ms, bound by
+// scalar and vector issue (1,900 and 1,060 instructions a stream) at 20 waves a
+// CU (24.3 ms with one lane encoding each stream).  Streams of a few values are
+// encoded by a thread each.  The scan and the interleave are the shared
+// lane-encoder kernels (lanes_enc_dev.h).
 #include <type_traits>
 
 #include "lanes_enc_dev.h"
