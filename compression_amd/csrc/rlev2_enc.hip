@@ -636,7 +636,7 @@ uint64_t v2_lane_slot(uint64_t chunk, uint32_t eb) {
 
 int rlev2_compress_bound(uint64_t in_bytes, uint64_t chunk, uint32_t eb, uint32_t ru, uint64_t* n_chunks,
                          uint64_t* work_bytes, uint64_t* payload_cap) {
-    if (!(eb == 1 || eb == 2 || eb == 4 || eb == 8) || ru == 0 || chunk % (32ull * eb) ||
+    if (!(eb == 1 || eb == 2 || eb == 4 || eb == 8) || ru == 0 || chunk == 0 || chunk % (32ull * eb) ||
         (chunk / eb / 32) % ru || in_bytes == 0 || chunk > (1ull << 32))
         return MDZ_ERR_INVALID;
     const uint64_t n = (in_bytes + chunk - 1) / chunk;

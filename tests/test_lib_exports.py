@@ -66,6 +66,7 @@ def test_encoder_bounds_checked_on_host():
     assert lib.mdz_rlev2_compress_bound(1 << 30, 131072, 8, 512, C.byref(n), C.byref(w), C.byref(p)) == 0
     assert n.value == 8192
     assert lib.mdz_rlev2_compress_bound(1000, 131072, 8, 3, C.byref(n), C.byref(w), C.byref(p)) == -1
+    assert lib.mdz_rlev2_compress_bound(1000, 0, 8, 4, C.byref(n), C.byref(w), C.byref(p)) == -1
     assert lib.mdz_brle_compress_bound(300_000, 262144, C.byref(n), C.byref(w), C.byref(p)) == 0
     assert n.value == 2 and p.value >= 300_000
     assert lib.mdz_brle_compress_bound(0, 262144, C.byref(n), C.byref(w), C.byref(p)) == -1
